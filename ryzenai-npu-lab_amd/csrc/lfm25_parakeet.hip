@@ -2,9 +2,9 @@
 // (experiments/pk_model.py, pk_engine.py, kernels/pk/pk_core.cc, pk_fast.cc)
 // as four kernels per block phase kind, one stream:
 //
-//   GEMM      C = bf16(epi(A . B + bias)) on the matrix cores, 128 x 128 block
-//             tiles (replaces gemm_step / pk_wx / epilogue,
-//             pk_fast.cc:167-231, pk_core.cc:169-183)
+//   GEMM      C = bf16(epi(A . B + bias)) on the matrix cores, 32 x 64 to
+//             128 x 128 block tiles (lfm25_gemm.h; replaces gemm_step / pk_wx /
+//             epilogue, pk_fast.cc:167-231, pk_core.cc:169-183)
 //   LN        scaled residual + LayerNorm (+ a second LayerNorm)
 //             (layer_norm / residual / ln_frame, pk_core.cc:55-116)
 //   ATT       relative-position attention of one (sequence, head)
@@ -25,6 +25,7 @@
 
 #include "lfm25_host.h"
 #include "lfm25_device.h"
+#include "lfm25_gemm.h"
 
 namespace lfm25 {
 namespace {
@@ -58,43 +59,17 @@ __device__ __forceinline__ float max_lanes16(float v) {
 
 // ------------------------------------------------------------------ GEMM
 
-// C[m][n] = bf16(epi(sum_k A[m][k] Bt[n][k] + bias[n])) for a (64 kWM) x 128
-// tile per block (blockIdx.x: n tile, blockIdx.y: m tile, blockIdx.z: batch
-// of independent products with element strides, or the K split). 2 kWM waves
-// in kWM x 2, each 64 x 64 as 4 x 4 MFMA tiles (v_mfma_f32_16x16x32_bf16 with
-// the weight tile as the first operand, so a lane's four results are four
-// consecutive n of one row m and leave as one 8-byte store). kWM = 2 (128 x
-// 128, two blocks per CU) by default; kWM = 4 (256 x 128, one block of 8
-// waves per CU) for wide products with many rows: the tile loads, which bound
-// this kernel through the L2 -> CU path, fall from 1/64 to 3/256 bytes per
-// FLOP. K steps of 64
-// go through double-buffered LDS: the next step's 16-byte global loads are
-// in flight in registers while the current step multiplies, and land in the
-// other buffer after it (one barrier per step). Rows m >= M read row M - 1
-// (their results are never stored), so every load is unconditional.
+// C[m][n] = bf16(epi(sum_k A[m][k] Bt[n][k] + bias[n])), one block tile per
+// block (lfm25_gemm.h; blockIdx.x: tile, blockIdx.y: K split). EPI_RESIDUAL: C = bf16(C + scale bf16(sum)), C the residual stream.
 //
 // Split K (kSplit): block z covers K range [z * kchunk, (z + 1) * kchunk) and
-// writes its FP32 partial tile to part[z][M][N]; k_pk_splitk sums the splits
-// in index order and applies the epilogue, so the result does not depend on
-// which blocks ran when.
-constexpr int kBM = 128, kBN = 128, kBK = 64;  // kBM: the tile height of split products
-// LDS holds each 64-wide K step of a tile row as eight 16-byte chunks; chunk
-// c of row r sits at position c ^ ((r / 2) % 8) of the row, so the 16-byte
-// reads of 16 consecutive rows at one chunk (an MFMA operand) and the
-// row-contiguous 16-byte stores both spread over all 64 banks (no bank
-// conflict cycles on gfx950; a one-chunk row padding leaves a third of the
-// LDS cycles in conflicts).
-constexpr int kRowChunks = 8;
-__device__ __forceinline__ int lds_chunk(int r, int c) { return r * kRowChunks + (c ^ ((r >> 1) & 7)); }
-constexpr int kSplitUnits = 256;  // split K until tiles x splits reaches this many blocks
-// ... or this many for products of at most 256 rows (one window): there the
-// FP32 partials of more splits cost more than the parallelism gains (a
-// 128-row tile writes as many partial bytes as it reads operand bytes)
-constexpr int kSplitUnitsFew = 64;
-constexpr int kMinChunk = 128;    // smallest K range of a split
-// FP32 partials: tiles x splits < 2 x kSplitUnits blocks of 128 x 128
-constexpr size_t kPartBytes = (size_t)2 * kSplitUnits * kBM * kBN * sizeof(float);
-enum PkEpi { EPI_NONE = 0, EPI_BIAS = 1, EPI_SWISH = 2 };
+// writes its FP32 partial tile to part[z][M][N]; k_pk_splitk or
+// k_pk_reduce_ln sums the splits in index order and applies the epilogue, so
+// the result does not depend on which blocks ran when.
+constexpr int kBN = 128;          // n is a multiple of this
+constexpr int kBK = tile::kStep;  // and k of this
+constexpr int kMinChunk = 512;    // smallest K range of a split
+enum PkEpi { EPI_NONE = 0, EPI_BIAS = 1, EPI_SWISH = 2, EPI_RESIDUAL = 3 };
 
 struct PkGemm {
   const uint16_t* A;
@@ -102,145 +77,67 @@ struct PkGemm {
   const uint16_t* bias;
   uint16_t* C;
   float* part;
-  long long sa, sb, sc;  // per-z element strides (batched products)
+  float scale;  // EPI_RESIDUAL
   int lda, ldb, ldc, M, N, kchunk;
+  bool wide;    // C and its rows are 16-byte aligned
+  tile::Tiles tiles;
 };
 
 template <int EPI>
 __device__ __forceinline__ float epilogue(float v, float b) {
   if (EPI == EPI_BIAS) v = v + b;
-  if (EPI == EPI_SWISH) v = v * sigmoid_f32(v);
+  if (EPI == EPI_SWISH) v = tile::over_one_plus_exp(v, v);
   return v;
 }
 
-// C = bf16(epi(A . B + bias)) per block tile of (64 kWM) x 128: kWM = 4 (256
-// rows, 8 waves) for the tall unsplit products, kWM = 2 (128 rows, 4 waves)
-// otherwise; each wave owns a 64 x 64 accumulator tile. The operands are
-// copied from global memory straight into LDS (global_load_lds, 16 bytes per
-// lane): no register staging and no LDS stores in the loop, three LDS stages
-// of one K step each (48 or 32 KB apiece), the copies of step s + 2 issued as
-// step s starts. A wave-instruction fills 64 consecutive 16-byte slots, so
-// each lane loads the chunk whose swizzled slot (lds_chunk) it fills. With
-// kSplit the block covers K range z and leaves its FP32 partial tile for
-// k_pk_splitk / k_pk_reduce_ln; rows past M read row M - 1 and are not
-// stored.
-typedef __attribute__((address_space(3))) void PkLdsVoid;
-typedef __attribute__((address_space(1))) void PkGlobalVoid;
-template <int kWM>
-struct PkGemmDmaLds {
-  uint4 a[3][64 * kWM * kRowChunks];
-  uint4 b[3][kBN * kRowChunks];
-};
-// One K step of 64 from LDS stage `buf` into the wave's 64 x 64 accumulators.
-template <int kWM>
-__device__ __forceinline__ void gemm_step_dma(const PkGemmDmaLds<kWM>& sh, int buf, int wm, int wn, int l,
-                                              f32x4_t (&acc)[4][4]) {
+template <int EPI, bool kSplit, typename S>
+__global__ void __launch_bounds__(S::kThreads, 2) k_pk_gemm(const PkGemm g) {
+  extern __shared__ __attribute__((aligned(16))) char lds_raw[];
+  auto& sh = *reinterpret_cast<tile::Lds<S>*>(lds_raw);
+  int tm, tn;
+  if (!g.tiles.of(blockIdx.x, tm, tn)) return;
+  const int n0 = tn * S::kTN, m0 = tm * S::kTM, z = blockIdx.y;
+  const size_t kbeg = kSplit ? (size_t)z * g.kchunk : 0;
+  tile::Copies<S> at;
+  tile::copy_offsets<S>(at, g.lda, g.ldb, [](int r) { return r; });
+  tile::Acc<S> acc;
+  acc.zero();
+  // a descriptor ends with the last row's last K element of this block's range
+  tile::product<S>(sh, g.A + (size_t)m0 * g.lda + kbeg,
+                   ((uint32_t)(min(S::kTM, g.M - m0) - 1) * g.lda + g.kchunk) * 2, g.Bt + (size_t)n0 * g.ldb + kbeg,
+                   ((uint32_t)(S::kTN - 1) * g.ldb + g.kchunk) * 2, at, g.kchunk / kBK, acc);
+  tile::each_row<S>(acc, m0, n0, g.M, [&](int m, int n, float (&v)[S::kLaneN]) {
+    if constexpr (kSplit) {
+      f32x4_t* p = reinterpret_cast<f32x4_t*>(g.part + ((size_t)z * g.M + m) * g.N + n);
 #pragma unroll
-  for (int ks = 0; ks < kBK / 32; ++ks) {
-    const int kc = 4 * ks + (l >> 4);  // chunk of k = 32 ks + 8 (l / 16) .. + 7
-    bf16x8_t xa[4], wb[4];
+      for (int i = 0; i < S::kLaneN / 4; ++i) p[i] = f32x4_t{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+    } else {
+      uint16_t* c = g.C + (size_t)m * g.ldc + n;
+      if constexpr (EPI == EPI_RESIDUAL) {
+        float x[S::kLaneN];
+        tile::load_bf16<S::kLaneN>(c, x);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      xa[i] = __builtin_bit_cast(bf16x8_t, sh.a[buf][lds_chunk(64 * wm + 16 * i + (l & 15), kc)]);
-      wb[i] = __builtin_bit_cast(bf16x8_t, sh.b[buf][lds_chunk(64 * wn + 16 * i + (l & 15), kc)]);
+        for (int i = 0; i < S::kLaneN; ++i) v[i] = x[i] + g.scale * round_bf16(v[i]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < S::kLaneN; ++i) v[i] = epilogue<EPI>(v[i], EPI == EPI_BIAS ? bf16_to_f32(g.bias[n + i]) : 0.0f);
+      }
+      tile::store_bf16<S::kLaneN>(c, v, g.wide);
     }
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
-        acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[nt], xa[mt], acc[nt][mt], 0, 0, 0);
-  }
+  });
 }
 
-template <int EPI, bool kSplit, int kWM>
-__global__ void __launch_bounds__(128 * kWM, 1) k_pk_gemm_dma(const PkGemm g) {
-  constexpr int kTileM = 64 * kWM;
-  constexpr int kAI = 4, kBI = 8 / kWM;  // copy instructions per wave and step: A, B
-  __shared__ PkGemmDmaLds<kWM> sh;
-  const int n0 = blockIdx.x * kBN, m0 = blockIdx.y * kTileM, z = blockIdx.z;
-  const int w = wave_id(), l = lane_id();
-  const int wm = w % kWM, wn = w / kWM;
-  const int kbeg = kSplit ? z * g.kchunk : 0;
-  const uint16_t* A = g.A + (kSplit ? 0 : g.sa * z) + kbeg;
-  const uint16_t* Bt = g.Bt + (kSplit ? 0 : g.sb * z) + kbeg;
-  // this lane's source rows and chunks: A slots (kAI w + i) * 64 + l, B slots (kBI w + i) * 64 + l
-  const uint16_t* pa[kAI];
-  const uint16_t* pb[kBI];
-#pragma unroll
-  for (int i = 0; i < kAI; ++i) {
-    const int p = (kAI * w + i) * kWave + l, r = p / kRowChunks, q = (p % kRowChunks) ^ ((r >> 1) & 7);
-    pa[i] = A + (size_t)min(m0 + r, g.M - 1) * g.lda + 8 * q;
-  }
-#pragma unroll
-  for (int i = 0; i < kBI; ++i) {
-    const int p = (kBI * w + i) * kWave + l, r = p / kRowChunks, q = (p % kRowChunks) ^ ((r >> 1) & 7);
-    pb[i] = Bt + (size_t)(n0 + r) * g.ldb + 8 * q;
-  }
-  const auto copy = [&](int step, int buf) {
-    const int k = step * kBK;
-#pragma unroll
-    for (int i = 0; i < kAI; ++i)
-      __builtin_amdgcn_global_load_lds((PkGlobalVoid*)(pa[i] + k), (PkLdsVoid*)&sh.a[buf][(kAI * w + i) * kWave], 16, 0,
-                                       0);
-#pragma unroll
-    for (int i = 0; i < kBI; ++i)
-      __builtin_amdgcn_global_load_lds((PkGlobalVoid*)(pb[i] + k), (PkLdsVoid*)&sh.b[buf][(kBI * w + i) * kWave], 16, 0,
-                                       0);
-  };
-  const int steps = g.kchunk / kBK;
-  f32x4_t acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  copy(0, 0);
-  if (steps > 1) copy(1, 1);
-  int buf = 0;
-  for (int s = 0; s < steps; ++s) {
-    // this wave's copies of step s have landed (those of step s + 1, kAI +
-    // kBI loads, may still be in flight); the barrier makes every wave's so,
-    // and puts every wave's reads of step s - 1's buffer behind it
-    if (s + 1 < steps) __builtin_amdgcn_s_waitcnt(0x0F70 | (kAI + kBI));  // vmcnt(kAI + kBI)
-    else __builtin_amdgcn_s_waitcnt(0x0F70);                              // vmcnt(0)
-    __builtin_amdgcn_s_barrier();
-    if (s + 2 < steps) copy(s + 2, buf == 0 ? 2 : buf - 1);
-    gemm_step_dma<kWM>(sh, buf, wm, wn, l, acc);
-    buf = buf == 2 ? 0 : buf + 1;
-  }
-  if (kSplit) {
-    float* P = g.part + (size_t)z * g.M * g.N;
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      const int n = n0 + 64 * wn + 16 * nt + 4 * (l >> 4);
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt) {
-        const int m = m0 + 64 * wm + 16 * mt + (l & 15);
-        if (m < g.M) *reinterpret_cast<f32x4_t*>(P + (size_t)m * g.N + n) = acc[nt][mt];
-      }
-    }
-    return;
-  }
-  uint16_t* C = g.C + g.sc * z;
-#pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
-    const int n = n0 + 64 * wn + 16 * nt + 4 * (l >> 4);
-    float bs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (EPI == EPI_BIAS) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) bs[e] = bf16_to_f32(g.bias[n + e]);
-    }
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-      const int m = m0 + 64 * wm + 16 * mt + (l & 15);
-      if (m >= g.M) continue;
-      u32x2_t pk;
-      pk.x = (uint32_t)f32_to_bf16(epilogue<EPI>(acc[nt][mt][0], bs[0])) |
-             ((uint32_t)f32_to_bf16(epilogue<EPI>(acc[nt][mt][1], bs[1])) << 16);
-      pk.y = (uint32_t)f32_to_bf16(epilogue<EPI>(acc[nt][mt][2], bs[2])) |
-             ((uint32_t)f32_to_bf16(epilogue<EPI>(acc[nt][mt][3], bs[3])) << 16);
-      *reinterpret_cast<u32x2_t*>(C + (size_t)m * g.ldc + n) = pk;
-    }
-  }
+// The same product where rows lie farther apart than a tile's 32-bit offsets
+// reach (kFarRows elements): an output per thread, 64-bit addresses.
+constexpr int kFarRows = 1 << 22;
+template <int EPI>
+__global__ void __launch_bounds__(256) k_pk_gemm_far(const PkGemm g) {
+  const int n = blockIdx.x * 256 + threadIdx.x, m = blockIdx.y;
+  if (n >= g.N) return;
+  const uint16_t *a = g.A + (size_t)m * g.lda, *b = g.Bt + (size_t)n * g.ldb;
+  float acc = 0.0f;
+  for (int k = 0; k < g.kchunk; ++k) acc = fmaf(bf16_to_f32(a[k]), bf16_to_f32(b[k]), acc);
+  g.C[(size_t)m * g.ldc + n] = f32_to_bf16(epilogue<EPI>(acc, EPI == EPI_BIAS ? bf16_to_f32(g.bias[n]) : 0.0f));
 }
 
 // y += partials z .. z + G - 1 of a thread's NQ x 4 values (partial i at
@@ -423,20 +320,19 @@ __global__ void __launch_bounds__(kLnRows* kWave) k_pk_ln(uint16_t* __restrict__
 // The end of a d-wide product whose `splits` FP32 partials sit in
 // part[z][rows][1024]: y = bf16(sum of the partials in index order), then
 // x' = bf16(x + s * y) and ln_modes (the GEMM's store, residual and
-// LayerNorm phases of pk_core.cc:90-116 in one pass over the row). R rows
-// (waves) per block: one when the product has few rows, so that a row's
-// splits x 4 KB of partials are spread over as many CUs as there are rows
-// (a CU's load rate, not HBM, bounds this pass).
-template <int R, int G>
-__global__ void __launch_bounds__(R* kWave) k_pk_reduce_ln(const float* __restrict__ part, int splits,
+// LayerNorm phases of pk_core.cc:90-116 in one pass over the row). One row
+// (wave) per block: only products of few rows are split, and a row's splits
+// x 4 KB of partials are then spread over as many CUs as there are rows (a
+// CU's load rate, not HBM, bounds this pass).
+template <int G>
+__global__ void __launch_bounds__(kWave) k_pk_reduce_ln(const float* __restrict__ part, int splits,
                                                                  uint16_t* __restrict__ x, float s,
                                                                  const uint16_t* __restrict__ g1,
                                                                  const uint16_t* __restrict__ b1,
                                                                  const uint16_t* __restrict__ g2,
                                                                  const uint16_t* __restrict__ b2, int normed_x,
                                                                  uint16_t* __restrict__ a, int rows) {
-  const int m = blockIdx.x * R + wave_id();
-  if (m >= rows) return;
+  const int m = blockIdx.x;
   const size_t off = (size_t)m * kD + 16 * lane_id();
   const size_t stride = (size_t)rows * kD;
   // the residual row and the norms' parameters first: in flight with the partials
@@ -778,31 +674,26 @@ __global__ void __launch_bounds__(kConvThreads) k_pk_conv(const uint16_t* __rest
 // ------------------------------------------------------------------ host
 
 // Number of K splits for an m x n x k product: doubled while the grid has
-// fewer than kSplitUnits (kSplitUnitsFew) blocks, each split keeping >=
-// kMinChunk of K.
-inline bool use_tall(int m, int n, int splits);
+// fewer blocks than the chip has CUs even with the smallest tile, each split
+// keeping >= kMinChunk of K. (128 x 1024 x 4096 alone: 11.1 us unsplit, 6.8 /
+// 4.8 / 4.9 in 2 / 4 / 8 splits; with K = 1024 4.5, 3.6 and 3.3 in 1, 2 and
+// 4, where the fourth partial costs the pass that sums them as much.)
 int pick_splits(int m, int n, int k) {
-  if (use_tall(m, n, 1)) return 1;
-  const int tiles = (n / kBN) * ((m + kBM - 1) / kBM);
   int splits = 1;
-  const int units = m <= 256 ? kSplitUnitsFew : kSplitUnits;
-  while (tiles * splits < units && k % (2 * splits * kBK) == 0 && k / (2 * splits) >= kMinChunk) splits *= 2;
+  while (tile::blocks_of<tile::S32x64>(m, n) * 2 * splits <= tile::kCus && k % (2 * splits * kBK) == 0 &&
+         k / (2 * splits) >= kMinChunk)
+    splits *= 2;
   return splits;
 }
 
-// Tall (256-row) tiles for an unsplit product with at least kTallTiles of
-// them: fewer bytes per FLOP, and still about one block per CU.
-constexpr int kTallTiles = 192;
-inline bool use_tall(int m, int n, int splits) {
-  return splits == 1 && (n / kBN) * ((m + 255) / 256) >= kTallTiles;
-}
-
-template <int EPI, int kWM>
-void launch_gemm(const PkGemm& g, dim3 grid, bool split, hipStream_t s) {
-  if (split)
-    k_pk_gemm_dma<EPI, true, kWM><<<grid, 128 * kWM, 0, s>>>(g);
-  else
-    k_pk_gemm_dma<EPI, false, kWM><<<grid, 128 * kWM, 0, s>>>(g);
+template <int EPI, bool kSplit>
+void launch_gemm(const PkGemm& g, int splits, hipStream_t s) {
+  tile::with_shape(g.M, g.N, splits, [&](auto shape) {
+    using S = decltype(shape);
+    PkGemm h = g;
+    h.tiles = tile::tiles_of<S>(g.M, g.N, (int64_t)g.M * g.kchunk * 2);
+    k_pk_gemm<EPI, kSplit, S><<<dim3(h.tiles.blocks(), splits), S::kThreads, sizeof(tile::Lds<S>), s>>>(h);
+  });
 }
 
 template <int EPI>
@@ -816,40 +707,45 @@ void launch_splitk(dim3 grid, const float* part, int splits, int m, int n, const
   }
 }
 
-// C = epi(A . Bt^T + bias) for `batch` products at element strides sa / sb /
-// sc, or (splits > 1, batch 1) as `splits` K ranges through `part`
-// (splits x m x n floats) and k_pk_splitk.
-int gemm(const uint16_t* a, int lda, long long sa, const uint16_t* bt, int ldb, long long sb, const uint16_t* bias,
-         uint16_t* c, int ldc, long long sc, int m, int n, int k, int batch, int epi, int splits, float* part,
-         hipStream_t s) {
-  const bool split = splits > 1;
-  const bool tall = batch == 1 && use_tall(m, n, splits);
-  const int tile_m = tall ? 256 : kBM;
-  const dim3 grid(n / kBN, (m + tile_m - 1) / tile_m, split ? splits : batch);
-  PkGemm g{a, bt, bias, c, part, sa, sb, sc, lda, ldb, ldc, m, n, k / splits};
-  switch (epi * 2 + (tall ? 1 : 0)) {
-    case 2 * EPI_NONE: launch_gemm<EPI_NONE, 2>(g, grid, split, s); break;
-    case 2 * EPI_NONE + 1: launch_gemm<EPI_NONE, 4>(g, grid, split, s); break;
-    case 2 * EPI_BIAS: launch_gemm<EPI_BIAS, 2>(g, grid, split, s); break;
-    case 2 * EPI_BIAS + 1: launch_gemm<EPI_BIAS, 4>(g, grid, split, s); break;
-    case 2 * EPI_SWISH: launch_gemm<EPI_SWISH, 2>(g, grid, split, s); break;
-    default: launch_gemm<EPI_SWISH, 4>(g, grid, split, s); break;
-  }
-  if (split) {
+// C = epi(A . Bt^T + bias), or (splits > 1) as `splits` K ranges through
+// `part` (splits x m x n floats) and k_pk_splitk.
+int gemm(const uint16_t* a, int lda, const uint16_t* bt, int ldb, const uint16_t* bias, uint16_t* c, int ldc, int m,
+         int n, int k, int epi, int splits, float* part, hipStream_t s) {
+  const bool wide = aligned16(c) && ldc % 8 == 0;
+  const PkGemm g{a, bt, bias, c, part, 0.0f, lda, ldb, ldc, m, n, k / splits, wide, {}};
+  if (lda > kFarRows || ldb > kFarRows) {
+    PkGemm f = g;
+    f.kchunk = k;
+    const dim3 grid((n + 255) / 256, m);
+    switch (epi) {
+      case EPI_NONE: k_pk_gemm_far<EPI_NONE><<<grid, 256, 0, s>>>(f); break;
+      case EPI_BIAS: k_pk_gemm_far<EPI_BIAS><<<grid, 256, 0, s>>>(f); break;
+      default: k_pk_gemm_far<EPI_SWISH><<<grid, 256, 0, s>>>(f); break;
+    }
+  } else if (splits > 1) {
+    launch_gemm<EPI_NONE, true>(g, splits, s);
     const dim3 blocks((unsigned)m, (unsigned)((n / 4 + 255) / 256));
     switch (epi) {
       case EPI_NONE: launch_splitk<EPI_NONE>(blocks, part, splits, m, n, bias, c, ldc, s); break;
       case EPI_BIAS: launch_splitk<EPI_BIAS>(blocks, part, splits, m, n, bias, c, ldc, s); break;
       default: launch_splitk<EPI_SWISH>(blocks, part, splits, m, n, bias, c, ldc, s); break;
     }
+  } else {
+    switch (epi) {
+      case EPI_NONE: launch_gemm<EPI_NONE, false>(g, 1, s); break;
+      case EPI_BIAS: launch_gemm<EPI_BIAS, false>(g, 1, s); break;
+      default: launch_gemm<EPI_SWISH, false>(g, 1, s); break;
+    }
   }
   return check_launch("parakeet gemm");
 }
 
-// One encoder product: split as pick_splits chooses, through the partial buffer.
+// One encoder product wider than d. Never split: at one window its smallest
+// tiles already fill half the chip, and the pass that sums the partials
+// would cost more than the other half gives.
 int enc_gemm(const uint16_t* a, int lda, const uint16_t* bt, const uint16_t* bias, uint16_t* c, int ldc, int m, int n,
-             int k, int epi, float* part, hipStream_t s) {
-  return gemm(a, lda, 0, bt, k, 0, bias, c, ldc, 0, m, n, k, 1, epi, pick_splits(m, n, k), part, s);
+             int k, int epi, hipStream_t s) {
+  return gemm(a, lda, bt, k, bias, c, ldc, m, n, k, epi, 1, nullptr, s);
 }
 
 struct ReduceLnArgs {
@@ -862,48 +758,42 @@ struct ReduceLnArgs {
   uint16_t* a;
   int rows;
 };
-template <int R, int G>
+template <int G>
 void launch_reduce_ln(const ReduceLnArgs& r, hipStream_t s) {
-  k_pk_reduce_ln<R, G><<<(r.rows + R - 1) / R, R * kWave, 0, s>>>(r.part, r.splits, r.x, r.scale, r.g1, r.b1, r.g2,
+  k_pk_reduce_ln<G><<<r.rows, kWave, 0, s>>>(r.part, r.splits, r.x, r.scale, r.g1, r.b1, r.g2,
                                                                    r.b2, r.normed_x, r.a, r.rows);
 }
 
 // A d-wide encoder product (m x 1024) whose end is a residual + LayerNorm:
-// its FP32 partial products (one per K split, at least one) go to `part`
-// and k_pk_reduce_ln finishes the row.
+// unsplit, the product's own epilogue updates x and k_pk_ln norms its rows;
+// split (few rows), the FP32 partials go to `part` and k_pk_reduce_ln
+// finishes the row.
 int enc_gemm_ln(const uint16_t* a, int lda, const uint16_t* bt, int m, int k, float* part, uint16_t* x, float scale,
                 const uint16_t* ln1, const uint16_t* ln2, int normed_x, uint16_t* out_a, hipStream_t s) {
   const int splits = pick_splits(m, kD, k);
-  const dim3 grid(kD / kBN, (m + kBM - 1) / kBM, splits);
-  PkGemm g{a, bt, nullptr, nullptr, part, 0, 0, 0, lda, k, kD, m, kD, k / splits};
-  k_pk_gemm_dma<EPI_NONE, true, 2><<<grid, 256, 0, s>>>(g);
-  const ReduceLnArgs r{part, splits, x, scale, ln1, ln1 + kD, ln2, ln2 ? ln2 + kD : nullptr, normed_x, out_a, m};
-  // A wave per block for few rows (latency-bound: all of a row's partials in
-  // flight at once); blocks of kLnRows waves, at most two partials per round
-  // trip, for many (a 16-window pass has two splits, and loading both at
-  // once measured 1.1% faster on the pass than one at a time)
-  if (m <= kSplitUnits) {
-    switch (partial_group(splits)) {
-      case 1: launch_reduce_ln<1, 1>(r, s); break;
-      case 2: launch_reduce_ln<1, 2>(r, s); break;
-      case 4: launch_reduce_ln<1, 4>(r, s); break;
-      default: launch_reduce_ln<1, 8>(r, s); break;
-    }
-  } else if (splits >= 2) {
-    launch_reduce_ln<kLnRows, 2>(r, s);
-  } else {
-    launch_reduce_ln<kLnRows, 1>(r, s);
+  const PkGemm g{a, bt, nullptr, x, part, scale, lda, k, kD, m, kD, k / splits, true, {}};
+  const uint16_t* b2 = ln2 ? ln2 + kD : nullptr;
+  if (splits == 1) {
+    launch_gemm<EPI_RESIDUAL, false>(g, 1, s);
+    k_pk_ln<<<(m + kLnRows - 1) / kLnRows, kLnRows * kWave, 0, s>>>(x, nullptr, 0.0f, ln1, ln1 + kD, ln2, b2, normed_x,
+                                                                    out_a, m);
+    return check_launch("parakeet gemm + layer norm");
   }
+  launch_gemm<EPI_NONE, true>(g, splits, s);
+  const ReduceLnArgs r{part, splits, x, scale, ln1, ln1 + kD, ln2, b2, normed_x, out_a, m};
+  // a wave per block: latency-bound, all of a row's partials in flight at once
+  if (splits == 2) launch_reduce_ln<2>(r, s);
+  else launch_reduce_ln<4>(r, s);
   return check_launch("parakeet gemm + layer norm");
 }
 
-// FP32 partial buffer of the encoder: split products stay under
-// 2 * kSplitUnits tiles; an unsplit d-wide product needs rows x 1024 floats.
-inline size_t pk_part_bytes(int rows) { return std::max(kPartBytes, (size_t)rows * kD * sizeof(float)); }
+// FP32 partial buffer of the encoder: split products (pick_splits) have at
+// most kCus blocks of the smallest tile.
+constexpr size_t kPartBytes = (size_t)tile::kCus * tile::S32x64::kTM * tile::S32x64::kTN * sizeof(float);
 
 // Workspace of the encoder for `rows` = batch * 128 frames (bytes).
 inline size_t pk_ws_bytes(int rows) {
-  return pk_part_bytes(rows) + (size_t)rows * 2 * (kD /*a*/ + kPkFfn /*big*/ + kD /*o*/);
+  return kPartBytes + (size_t)rows * 2 * (kD /*a*/ + kPkFfn /*big*/ + kD /*o*/);
 }
 
 }  // namespace
@@ -929,7 +819,7 @@ int lfm25_pk_gemm(const uint16_t* a, int32_t lda, const uint16_t* bt, int32_t ld
                 "pk gemm: splits must divide k into multiples of %d (got %d splits of %d)", kBK, splits, k);
   LFM25_REQUIRE(splits == 1 || (workspace && aligned16(workspace)),
                 "pk gemm: a split product needs a 16-byte aligned workspace of splits * m * n floats");
-  return gemm(a, lda, 0, bt, ldb, 0, bias, c, ldc, 0, m, n, k, 1, epi, splits, static_cast<float*>(workspace),
+  return gemm(a, lda, bt, ldb, bias, c, ldc, m, n, k, epi, splits, static_cast<float*>(workspace),
               reinterpret_cast<hipStream_t>(stream));
 }
 
@@ -996,7 +886,7 @@ int lfm25_pk_encoder(const lfm25_pk_layer* layers, int32_t n_layers, uint16_t* x
   const int rows = batch * frames;
   char* ws = static_cast<char*>(workspace);
   float* part = reinterpret_cast<float*>(ws);
-  uint16_t* a = reinterpret_cast<uint16_t*>(ws + pk_part_bytes(rows));
+  uint16_t* a = reinterpret_cast<uint16_t*>(ws + kPartBytes);
   uint16_t* big = a + (size_t)rows * kD;
   uint16_t* o = big + (size_t)rows * kPkFfn;
   int rc = LFM25_OK;
@@ -1015,19 +905,19 @@ int lfm25_pk_encoder(const lfm25_pk_layer* layers, int32_t n_layers, uint16_t* x
     const lfm25_pk_layer& L = layers[i];
     const uint16_t* next_ln = i + 1 < n_layers ? ln_of(layers[i + 1], 0) : nullptr;
     // Macaron FFN 1: x = bf16(x + FFN(a) / 2), a = LN_att(x)
-    PK_TRY(enc_gemm(a, kD, L.ff1_w1, nullptr, big, kPkFfn, rows, kPkFfn, kD, EPI_SWISH, part, s));
+    PK_TRY(enc_gemm(a, kD, L.ff1_w1, nullptr, big, kPkFfn, rows, kPkFfn, kD, EPI_SWISH, s));
     PK_TRY(enc_gemm_ln(big, kPkFfn, L.ff1_w2, rows, kPkFfn, part, x, 0.5f, ln_of(L, 1), nullptr, 0, a, s));
     // relative-position self-attention: x = bf16(x + out(att)), a = LN_conv(x)
-    PK_TRY(enc_gemm(a, kD, L.qkv, L.qkv_bias, big, 3 * kD, rows, 3 * kD, kD, EPI_BIAS, part, s));
+    PK_TRY(enc_gemm(a, kD, L.qkv, L.qkv_bias, big, 3 * kD, rows, 3 * kD, kD, EPI_BIAS, s));
     k_pk_attention<<<dim3(kPkHeads, batch, kAttSplit), kAttBlockThreads, 0, s>>>(big, L.pos, L.att_delta, o, valid);
     PK_TRY(enc_gemm_ln(o, kD, L.out, rows, kD, part, x, 1.0f, ln_of(L, 2), nullptr, 0, a, s));
     // conv module: x = bf16(x + pw2(conv(pw1(a)))), a = LN_ff2(x)
-    PK_TRY(enc_gemm(a, kD, L.pw1, nullptr, big, 2 * kD, rows, 2 * kD, kD, EPI_NONE, part, s));
+    PK_TRY(enc_gemm(a, kD, L.pw1, nullptr, big, 2 * kD, rows, 2 * kD, kD, EPI_NONE, s));
     k_pk_conv<<<dim3(kD / kConvCh, batch), kConvThreads, 0, s>>>(big, L.dw, L.dw_b, o, valid);
     PK_TRY(enc_gemm_ln(o, kD, L.pw2, rows, kD, part, x, 1.0f, ln_of(L, 3), nullptr, 0, a, s));
     // Macaron FFN 2 and the block's output norm: x = LN_out(bf16(x + FFN(a) / 2)),
     // a = LN_ff1 of the next layer (x)
-    PK_TRY(enc_gemm(a, kD, L.ff2_w1, nullptr, big, kPkFfn, rows, kPkFfn, kD, EPI_SWISH, part, s));
+    PK_TRY(enc_gemm(a, kD, L.ff2_w1, nullptr, big, kPkFfn, rows, kPkFfn, kD, EPI_SWISH, s));
     PK_TRY(enc_gemm_ln(big, kPkFfn, L.ff2_w2, rows, kPkFfn, part, x, 0.5f, ln_of(L, 4), next_ln, 1, a, s));
   }
 #undef PK_TRY
