@@ -41,8 +41,6 @@ constexpr int kPkFfn = 4096;
 constexpr int kConvTapsPk = 9;
 constexpr float kLnEps = 1.0e-5f;
 
-__device__ __forceinline__ float sigmoid_f32(float x) { return 1.0f / (1.0f + expf(-x)); }
-
 // Sum / maximum over the four lanes l, l ^ 16, l ^ 32, l ^ 48 (gfx950 row swaps).
 __device__ __forceinline__ float sum_lanes16(float v) {
   const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -593,82 +591,86 @@ __global__ void __launch_bounds__(kAttBlockThreads, 1)
 
 // ------------------------------------------------------------------ conv module
 
-// GLU + depthwise conv of 16 channels (blockIdx.x) of sequence b
-// (blockIdx.y), as the mirror (012_layer_test.py:92-100):
+// GLU + depthwise conv of 64 channels (blockIdx.x) over 32 frames
+// (blockIdx.y) of sequence b (blockIdx.z), as the mirror
+// (012_layer_test.py:92-100):
 //   g_t = bf16(c_t[ch] * sigmoid(c_t[1024 + ch])) for t < valid, else 0;
 //   y_t = sum_{j<9} g_{t+j-4} * dw[ch][j] (in order, zero outside the
 //   frames) + bias[ch]; out = bf16(y * sigmoid(y)).
-// A thread handles 8 adjacent channels: 16-byte loads of the GLU halves and
-// the taps, 16-byte output stores. (16 channels a block: at one window that
-// is 64 blocks, and a thread's GLU loads take about one round trip; with 64
-// channels a block the 16 blocks' threads chained four or five.)
-constexpr int kConvCh = 16;
+// Eight threads side by side take 64 adjacent channels of a frame, so every
+// load and store covers whole 128-byte lines (with 16 channels a block they
+// were 32-byte pieces of a 4 KB row, which bound the pass: 12.2 us at 16
+// windows); the four frames to either side are formed twice.
+constexpr int kConvCh = 64;
+constexpr int kConvFrames = 32;
 constexpr int kConvThreads = 256;
+static_assert(kConvThreads == kConvFrames * kConvCh / 8, "a frame's eight channels per thread");
 __global__ void __launch_bounds__(kConvThreads) k_pk_conv(const uint16_t* __restrict__ c, const uint16_t* __restrict__ dw,
                                                           const uint16_t* __restrict__ dw_b,
                                                           uint16_t* __restrict__ out, int valid) {
-  __shared__ float g[kAttT + 8][kConvCh];
-  const int ch0 = blockIdx.x * kConvCh, b = blockIdx.y, t = threadIdx.x;
-  for (int e = t; e < (kAttT + 8) * (kConvCh / 8); e += kConvThreads) {
-    const int tt = e / (kConvCh / 8) - 4, q = e % (kConvCh / 8);
+  constexpr int kHalo = kConvTapsPk / 2, kRows = kConvFrames + 2 * kHalo;
+  __shared__ float g[kRows][kConvCh + 4];
+  const int ch0 = blockIdx.x * kConvCh, t0 = blockIdx.y * kConvFrames, b = blockIdx.z, t = threadIdx.x;
+  // this thread's channels ch0 + 8q .. + 7 and frame t0 + r
+  const int q = t % (kConvCh / 8), r = t / (kConvCh / 8);
+  const int ch = ch0 + 8 * q;
+  const uint4* taps = reinterpret_cast<const uint4*>(dw + (size_t)ch * kConvTapsPk);  // 72 values, 9 x 16 bytes
+  uint4 tap[kConvTapsPk];
+#pragma unroll
+  for (int u = 0; u < kConvTapsPk; ++u) tap[u] = taps[u];
+  const uint4 bv = *reinterpret_cast<const uint4*>(dw_b + ch);
+  // the GLU of rows r and (the last 8) r + 32; row i is frame t0 + i - 4
+  const auto glu = [&](int i) {
+    const int tt = t0 + i - kHalo;
     float v[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     if (tt >= 0 && tt < valid) {
-      const uint16_t* row = c + (size_t)(b * kAttT + tt) * 2 * kD + ch0 + 8 * q;
+      const uint16_t* row = c + (size_t)(b * kAttT + tt) * 2 * kD + ch;
       const uint4 av = *reinterpret_cast<const uint4*>(row);
       const uint4 gv = *reinterpret_cast<const uint4*>(row + kD);
       const uint32_t aw[4] = {av.x, av.y, av.z, av.w}, gw[4] = {gv.x, gv.y, gv.z, gv.w};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        v[2 * i] = round_bf16(lo_f32(aw[i]) * sigmoid_f32(lo_f32(gw[i])));
-        v[2 * i + 1] = round_bf16(hi_f32(aw[i]) * sigmoid_f32(hi_f32(gw[i])));
+      for (int e = 0; e < 4; ++e) {
+        v[2 * e] = round_bf16(tile::over_one_plus_exp(lo_f32(aw[e]), lo_f32(gw[e])));
+        v[2 * e + 1] = round_bf16(tile::over_one_plus_exp(hi_f32(aw[e]), hi_f32(gw[e])));
       }
     }
-    float4* dst = reinterpret_cast<float4*>(&g[tt + 4][8 * q]);
+    float4* dst = reinterpret_cast<float4*>(&g[i][8 * q]);
     dst[0] = float4{v[0], v[1], v[2], v[3]};
     dst[1] = float4{v[4], v[5], v[6], v[7]};
-  }
-  // this thread's channels ch0 + 8q .. + 7: taps [8][9] and bias
-  const int q = t % (kConvCh / 8);
-  const int ch = ch0 + 8 * q;
+  };
+  glu(r);
+  if (r < 2 * kHalo) glu(r + kConvFrames);
   float wt[8][kConvTapsPk], bias[8];
-  {
-    const uint4* src = reinterpret_cast<const uint4*>(dw + (size_t)ch * kConvTapsPk);  // 72 values, 9 x 16 bytes
 #pragma unroll
-    for (int u = 0; u < kConvTapsPk; ++u) {
-      const uint4 v = src[u];
-      const uint32_t vw[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i0 = 8 * u + 2 * e;
-        wt[i0 / kConvTapsPk][i0 % kConvTapsPk] = lo_f32(vw[e]);
-        wt[(i0 + 1) / kConvTapsPk][(i0 + 1) % kConvTapsPk] = hi_f32(vw[e]);
-      }
-    }
-    const uint4 bv = *reinterpret_cast<const uint4*>(dw_b + ch);
-    const uint32_t bw[4] = {bv.x, bv.y, bv.z, bv.w};
+  for (int u = 0; u < kConvTapsPk; ++u) {
+    const uint32_t vw[4] = {tap[u].x, tap[u].y, tap[u].z, tap[u].w};
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      bias[2 * e] = lo_f32(bw[e]);
-      bias[2 * e + 1] = hi_f32(bw[e]);
+      const int i0 = 8 * u + 2 * e;
+      wt[i0 / kConvTapsPk][i0 % kConvTapsPk] = lo_f32(vw[e]);
+      wt[(i0 + 1) / kConvTapsPk][(i0 + 1) % kConvTapsPk] = hi_f32(vw[e]);
     }
+  }
+  const uint32_t bw[4] = {bv.x, bv.y, bv.z, bv.w};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    bias[2 * e] = lo_f32(bw[e]);
+    bias[2 * e + 1] = hi_f32(bw[e]);
   }
   __syncthreads();
-  for (int tt = t / (kConvCh / 8); tt < kAttT; tt += kConvThreads / (kConvCh / 8)) {
-    float y[8];
+  float y[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) y[k] = g[tt][8 * q + k] * wt[k][0];
+  for (int k = 0; k < 8; ++k) y[k] = g[r][8 * q + k] * wt[k][0];
 #pragma unroll
-    for (int j = 1; j < kConvTapsPk; ++j)
+  for (int j = 1; j < kConvTapsPk; ++j)
 #pragma unroll
-      for (int k = 0; k < 8; ++k) y[k] = y[k] + g[tt + j][8 * q + k] * wt[k][j];
-    uint32_t o[4];
+    for (int k = 0; k < 8; ++k) y[k] = y[k] + g[r + j][8 * q + k] * wt[k][j];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float y0 = y[2 * e] + bias[2 * e], y1 = y[2 * e + 1] + bias[2 * e + 1];
-      o[e] = (uint32_t)f32_to_bf16(y0 * sigmoid_f32(y0)) | ((uint32_t)f32_to_bf16(y1 * sigmoid_f32(y1)) << 16);
-    }
-    *reinterpret_cast<uint4*>(out + (size_t)(b * kAttT + tt) * kD + ch) = uint4{o[0], o[1], o[2], o[3]};
+  for (int k = 0; k < 8; ++k) {
+    y[k] = y[k] + bias[k];
+    y[k] = tile::over_one_plus_exp(y[k], y[k]);
   }
+  tile::store_bf16<8>(out + (size_t)(b * kAttT + t0 + r) * kD + ch, y, true);
 }
 
 // ------------------------------------------------------------------ host
@@ -855,7 +857,7 @@ int lfm25_pk_conv(const uint16_t* c, const uint16_t* dw, const uint16_t* dw_b, u
   LFM25_REQUIRE(frames == kAttT, "pk conv: frames must be %d, got %d", kAttT, frames);
   LFM25_REQUIRE(batch >= 1 && valid >= 1 && valid <= frames, "pk conv: need batch >= 1 and 1 <= valid <= frames");
   LFM25_REQUIRE(aligned16(c) && aligned16(dw) && aligned16(dw_b) && aligned16(out), "pk conv: 16-byte alignment");
-  k_pk_conv<<<dim3(kD / kConvCh, batch), kConvThreads, 0, reinterpret_cast<hipStream_t>(stream)>>>(c, dw, dw_b, out,
+  k_pk_conv<<<dim3(kD / kConvCh, kAttT / kConvFrames, batch), kConvThreads, 0, reinterpret_cast<hipStream_t>(stream)>>>(c, dw, dw_b, out,
                                                                                                    valid);
   return check_launch("parakeet conv");
 }
@@ -913,7 +915,7 @@ int lfm25_pk_encoder(const lfm25_pk_layer* layers, int32_t n_layers, uint16_t* x
     PK_TRY(enc_gemm_ln(o, kD, L.out, rows, kD, part, x, 1.0f, ln_of(L, 2), nullptr, 0, a, s));
     // conv module: x = bf16(x + pw2(conv(pw1(a)))), a = LN_ff2(x)
     PK_TRY(enc_gemm(a, kD, L.pw1, nullptr, big, 2 * kD, rows, 2 * kD, kD, EPI_NONE, s));
-    k_pk_conv<<<dim3(kD / kConvCh, batch), kConvThreads, 0, s>>>(big, L.dw, L.dw_b, o, valid);
+    k_pk_conv<<<dim3(kD / kConvCh, kAttT / kConvFrames, batch), kConvThreads, 0, s>>>(big, L.dw, L.dw_b, o, valid);
     PK_TRY(enc_gemm_ln(o, kD, L.pw2, rows, kD, part, x, 1.0f, ln_of(L, 3), nullptr, 0, a, s));
     // Macaron FFN 2 and the block's output norm: x = LN_out(bf16(x + FFN(a) / 2)),
     // a = LN_ff1 of the next layer (x)
