@@ -466,6 +466,23 @@ size_t lfm25_batch_workspace_bytes(void);
 int lfm25_batch_pass(const lfm25_batch* b, const int32_t* rows, int32_t n_rows, int32_t select,
                      int32_t* tokens_out, uint16_t* hidden_out, lfm25_stream_t stream);
 
+/* A prompt pass: up to LFM25_PROMPT_MAX_ROWS rows of one or more prompts
+ * through the model as matrix-matrix products, on the same caches, conv
+ * states and rounding points as lfm25_batch_pass (sums in another FP32
+ * order). runs: host int32 [n_runs][3], (sequence, position, count) of
+ * consecutive rows of a sequence, each sequence at most once, n_runs <=
+ * LFM25_BATCH_MAX_ROWS; tokens: device int32, the runs' rows in order.
+ * tokens_out (device int32 [n_runs], or NULL): the selection of each run's
+ * last row; hidden_out (device BF16 [n_runs x 1024], or NULL): its last
+ * layer's output. prompt_workspace: lfm25_prompt_workspace_bytes(rows) bytes,
+ * 16-byte aligned, contents ignored. Status flags as lfm25_batch_pass.
+ * Replaces prefill_design (experiments/lfm25_x8.py:341-416), which takes PB
+ * = 4 rows. */
+#define LFM25_PROMPT_MAX_ROWS 4096
+size_t lfm25_prompt_workspace_bytes(int32_t rows);
+int lfm25_prompt_pass(const lfm25_batch* b, const int32_t* tokens, const int32_t* runs, int32_t n_runs,
+                      int32_t* tokens_out, uint16_t* hidden_out, void* prompt_workspace, lfm25_stream_t stream);
+
 /* n_steps greedy steps of all b->sequences sequences in lockstep: at step i
  * sequence s consumes a token at position positions[s] + i (positions: host
  * int32 [sequences]) -- tokens_in[s] (device) at step 0, its own selection

@@ -53,6 +53,7 @@ class W8Model(ctypes.Structure):
 
 
 BATCH_MAX_ROWS = 64
+PROMPT_MAX_ROWS = 4096
 LAYER_CONV, LAYER_ATTN = 0, 1
 
 
@@ -117,6 +118,8 @@ SIGNATURES = {
     "lfm25_decode_w8": (ctypes.c_int, [ctypes.POINTER(Decoder), ctypes.POINTER(W8Model), _p, _i32, _i32, _p, _p]),
     "lfm25_batch_workspace_bytes": (_size, []),
     "lfm25_batch_pass": (ctypes.c_int, [ctypes.POINTER(Batch), _p, _i32, _i32, _p, _p, _p]),
+    "lfm25_prompt_workspace_bytes": (_size, [_i32]),
+    "lfm25_prompt_pass": (ctypes.c_int, [ctypes.POINTER(Batch), _p, _p, _i32, _p, _p, _p, _p]),
     "lfm25_batch_decode": (ctypes.c_int, [ctypes.POINTER(Batch), _p, _p, _i32, _p, _p]),
     "lfm25_batch_decode_hidden": (ctypes.c_int, [ctypes.POINTER(Batch), _p, _p, _i32, _p, _p, _p]),
     "lfm25_batch_linear": (ctypes.c_int, [_p, _p, _p, _i32, _i32, _i32, _p]),

@@ -48,6 +48,44 @@ def run_pass(desc: _lib.Batch, rows: list[tuple[int, int, int]], select: bool, t
               hidden_out.data_ptr() if hidden_out is not None else None, stream)
 
 
+# Rows from which one sequence's prompt takes a prompt pass (lfm25_prompt_pass)
+# instead of passes of up to MAX_ROWS rows: one pass of 64 rows takes 0.57 ms
+# and a prompt pass of 64 rows 0.62, of 96 rows 0.63, of 512 rows 0.84.
+PROMPT_ROWS = MAX_ROWS + 1
+# ... and a batch's prompts: up to four passes' rows keep the passes, which
+# give a row the same bits as run_rows does (a prompt pass sums in another
+# order). Four passes of 64 rows take 2.3 ms, a prompt pass of 256 rows 0.72.
+BATCH_PROMPT_ROWS = 4 * MAX_ROWS + 1
+
+
+class PromptWorkspace:
+    """The scratch memory of a model's prompt passes: kept between calls, at
+    the size of the longest prompt so far (at most lfm25_prompt_workspace_bytes
+    of PROMPT_MAX_ROWS rows, 50 MB), and given back with the model. The callers
+    wait for a pass before they return, so no stream still uses a buffer that
+    a longer prompt replaces."""
+
+    def __init__(self, device):
+        self.device = device
+        self._buffer = None
+
+    def pointer(self, rows: int) -> int:
+        need = int(_lib.load().lfm25_prompt_workspace_bytes(rows))
+        if self._buffer is None or self._buffer.numel() < need:
+            self._buffer = torch.empty(need, dtype=torch.uint8, device=self.device)
+        return self._buffer.data_ptr()
+
+
+def run_prompt(desc: _lib.Batch, workspace: PromptWorkspace, tokens: torch.Tensor, runs: list[tuple[int, int, int]],
+               tokens_out: torch.Tensor | None, stream: int) -> None:
+    """One lfm25_prompt_pass over `runs` = [(sequence, position, count), ...]
+    of the device token ids `tokens`."""
+    table = np.ascontiguousarray(np.asarray(runs, dtype=np.int32).reshape(-1, 3))
+    _lib.call("lfm25_prompt_pass", ctypes.byref(desc), tokens.data_ptr(), table.ctypes.data, len(table),
+              tokens_out.data_ptr() if tokens_out is not None else None, None,
+              workspace.pointer(int(table[:, 2].sum())), stream)
+
+
 class BatchDecoder:
     """B independent sequences decoded in lockstep on shared weights.
 
@@ -93,6 +131,7 @@ class BatchDecoder:
         self.values = torch.zeros(kv, **bf)
         self.workspace = torch.zeros(lib.lfm25_batch_workspace_bytes(), dtype=torch.uint8, device=self.device)
         self._tokens = torch.zeros(MAX_ROWS, dtype=torch.int32, device=self.device)
+        self._prompt_ws = PromptWorkspace(self.device)
         self._desc = _lib.Batch(self.weights.data_ptr(), self.table.data_ptr(), self.rope.data_ptr(),
                                 self.conv_states.data_ptr(), self.keys.data_ptr(), self.values.data_ptr(),
                                 self.workspace.data_ptr(), sequences, capacity, self.vocab)
@@ -151,16 +190,45 @@ class BatchDecoder:
                 raise ValueError(f"prompt {s} is empty")
             if self.positions[s] + len(p) > self.capacity:
                 raise ValueError(f"KV capacity {self.capacity} reached")
+        for s, p in pending:
+            for t in p:
+                if not 0 <= t < self.vocab:
+                    raise ValueError(f"token id {t} outside the vocabulary")
         nxt = [0] * self.sequences
-        queue = [(s, i, t) for s, p in pending for i, t in enumerate(p)]
-        start = list(self.positions)
-        while queue:
-            chunk, queue = queue[:MAX_ROWS], queue[MAX_ROWS:]
-            rows = [(t, s, start[s] + i) for s, i, t in chunk]
-            tokens, _ = self.run_rows(rows, select=True)
-            for (s, i, _), tok in zip(chunk, tokens):
-                if i == len(prompts[s]) - 1:
-                    nxt[s] = tok
+        if sum(len(p) for _, p in pending) < BATCH_PROMPT_ROWS:
+            rows = [(t, s, self.positions[s] + i) for s, p in pending for i, t in enumerate(p)]
+            ends = {(s, self.positions[s] + len(p) - 1) for s, p in pending}
+            for i in range(0, len(rows), MAX_ROWS):
+                chunk = rows[i:i + MAX_ROWS]
+                tokens, _ = self.run_rows(chunk, select=True)
+                for (_, s, pos), tok in zip(chunk, tokens):
+                    if (s, pos) in ends:
+                        nxt[s] = tok
+            return nxt
+        # prompt passes of up to PROMPT_MAX_ROWS rows, a prompt that does not
+        # fit the rest of one cut there; a run's selection counts where its
+        # prompt ends
+        ids = torch.tensor([t for _, p in pending for t in p], dtype=torch.int32).to(self.device)
+        done, at = [0] * self.sequences, 0
+        while at < ids.numel():
+            runs, room = [], _lib.PROMPT_MAX_ROWS
+            for s, p in pending:
+                take = min(len(p) - done[s], room)
+                if take > 0:
+                    runs.append((s, self.positions[s], take))
+                    room -= take
+            count = _lib.PROMPT_MAX_ROWS - room
+            run_prompt(self._desc, self._prompt_ws, ids[at:at + count], runs, self._tokens, self._stream())
+            at += count
+            for s, _, take in runs:
+                done[s] += take
+                self.positions[s] += take
+            tokens = self._tokens[:len(runs)].cpu().tolist()
+            if self._status():
+                raise RuntimeError(f"prompt pass ended with status 0x{self._status():x}")
+            for (s, _, _), tok in zip(runs, tokens):
+                if done[s] == len(pending[s][1]):
+                    nxt[s] = int(tok)
         return nxt
 
     def decode(self, tokens: list[int], n_steps: int) -> np.ndarray:

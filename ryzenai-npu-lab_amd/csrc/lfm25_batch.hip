@@ -802,6 +802,18 @@ __global__ void k_bx_set_starts(BatchParams p, StartTable t) {
   if ((int)threadIdx.x < p.seqs) reinterpret_cast<int32_t*>(p.ws + kBwStart)[threadIdx.x] = t.pos[threadIdx.x];
 }
 
+// The last rows of a prompt pass's runs: row r of X (and of `hidden`, if
+// given) = the last row of run r.
+__global__ void __launch_bounds__(kHidden / 8) k_bx_last_rows(BatchParams p, PromptRuns runs,
+                                                              const uint16_t* __restrict__ rows,
+                                                              uint16_t* __restrict__ hidden) {
+  int end = 0;
+  for (int r = 0; r <= (int)blockIdx.x; ++r) end += runs.run[r].count;
+  const uint4 v = reinterpret_cast<const uint4*>(rows + (size_t)(end - 1) * kHidden)[threadIdx.x];
+  reinterpret_cast<uint4*>(b_x(p) + (size_t)blockIdx.x * kHidden)[threadIdx.x] = v;
+  if (hidden != nullptr) reinterpret_cast<uint4*>(hidden + (size_t)blockIdx.x * kHidden)[threadIdx.x] = v;
+}
+
 // Y[m][n] = bf16(W[n] . X[m]) for the batch linear test entry point.
 template <int K>
 __global__ void __launch_bounds__(kGT) k_bx_linear(const uint16_t* x, const uint16_t* w, uint16_t* y, int rows, int n) {
@@ -819,6 +831,17 @@ __global__ void __launch_bounds__(kGT) k_bx_linear(const uint16_t* x, const uint
 // ------------------------------------------------------------------ host
 
 uint16_t* b_g_host(const BatchParams& p) { return reinterpret_cast<uint16_t*>(p.ws + kBwG); }
+
+// The final norm, the head and the picks of the rows of X.
+int launch_head(const BatchParams& p, int32_t* tokens_out, hipStream_t s) {
+  const int blocks = std::min(kHeadBlocks, (p.vocab + kHeadChunk - 1) / kHeadChunk);
+  if (p.rows > kFoldRows)
+    k_bx_norm<<<p.rows, 2 * kWave, 0, s>>>(p, reinterpret_cast<uint16_t*>(p.ws + kBwX), p.weights + layer_off(kLayers),
+                                           reinterpret_cast<uint16_t*>(p.ws + kBwXn));
+  k_bx_head<<<blocks, kGT, 0, s>>>(p);
+  k_bx_pick<<<p.rows, kAT, 0, s>>>(p, blocks, tokens_out);
+  return check_launch("batch head");
+}
 
 // (decode_tokens != nullptr: a decode step, whose row table the embedding
 // kernel writes: sequence m consumes decode_tokens[m] at its start + step.)
@@ -855,14 +878,7 @@ int launch_pass(const BatchParams& p, bool select, int32_t* tokens_out, uint16_t
   if (hidden_out != nullptr &&
       hipMemcpyAsync(hidden_out, x, (size_t)p.rows * kHidden * 2, hipMemcpyDeviceToDevice, s) != hipSuccess)
     return set_error(LFM25_EDEVICE, "batch pass: hidden copy failed");
-  if (select) {
-    const int blocks = std::min(kHeadBlocks, (p.vocab + kHeadChunk - 1) / kHeadChunk);
-    if (!fold) k_bx_norm<<<p.rows, 2 * kWave, 0, s>>>(p, x, p.weights + layer_off(kLayers), xn);
-    k_bx_head<<<blocks, kGT, 0, s>>>(p);
-    k_bx_pick<<<p.rows, kAT, 0, s>>>(p, blocks, tokens_out);
-    rc = check_launch("batch head");
-  }
-  return rc;
+  return select ? launch_head(p, tokens_out, s) : rc;
 }
 
 int check_batch(const lfm25_batch* b) {
@@ -937,6 +953,47 @@ int lfm25_batch_pass(const lfm25_batch* b, const int32_t* rows, int32_t n_rows, 
   k_bx_set_rows<<<1, kRowsMax, 0, s>>>(p, table);
   k_bx_status_clear<<<1, kHidden / 16, 0, s>>>(p, 1);
   return launch_pass(p, select != 0, tokens_out, hidden_out, s);
+}
+
+size_t lfm25_prompt_workspace_bytes(int32_t rows) {
+  return rows >= 1 && rows <= LFM25_PROMPT_MAX_ROWS ? prompt_bytes(rows) : 0;
+}
+
+int lfm25_prompt_pass(const lfm25_batch* b, const int32_t* tokens, const int32_t* runs, int32_t n_runs,
+                      int32_t* tokens_out, uint16_t* hidden_out, void* prompt_workspace, lfm25_stream_t stream) {
+  int rc = check_batch(b);
+  if (rc != LFM25_OK) return rc;
+  LFM25_REQUIRE(tokens != nullptr && runs != nullptr && prompt_workspace != nullptr, "prompt pass: null argument");
+  LFM25_REQUIRE(n_runs >= 1 && n_runs <= kRowsMax, "prompt pass: runs must be 1..%d, got %d", kRowsMax, n_runs);
+  LFM25_REQUIRE(aligned16(prompt_workspace) && aligned16(b->rope) && aligned16(b->key_cache) &&
+                    aligned16(b->value_cache) && (hidden_out == nullptr || aligned16(hidden_out)),
+                "prompt pass: workspace, rope, caches and hidden_out must be 16-byte aligned");
+  PromptRuns table{};
+  table.n = n_runs;
+  bool seen[kRowsMax] = {};
+  int64_t rows = 0;
+  for (int r = 0; r < n_runs; ++r) {
+    const PromptRun run{runs[3 * r], runs[3 * r + 1], runs[3 * r + 2]};
+    LFM25_REQUIRE(run.sequence >= 0 && run.sequence < b->sequences, "prompt pass: run %d sequence %d out of range", r,
+                  run.sequence);
+    LFM25_REQUIRE(!seen[run.sequence], "prompt pass: sequence %d appears in two runs", run.sequence);
+    LFM25_REQUIRE(run.position >= 0 && run.count >= 1 && run.count <= b->capacity - run.position,
+                  "prompt pass: run %d of %d rows at position %d does not fit the capacity %d", r, run.count,
+                  run.position, b->capacity);
+    seen[run.sequence] = true;
+    rows += run.count;
+    table.run[r] = run;
+  }
+  LFM25_REQUIRE(rows <= LFM25_PROMPT_MAX_ROWS, "prompt pass: %lld rows, at most %d", (long long)rows,
+                LFM25_PROMPT_MAX_ROWS);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const BatchParams p = make_batch_params(b, n_runs);
+  k_bx_status_clear<<<1, kHidden / 16, 0, s>>>(p, 1);
+  const uint16_t* x = nullptr;
+  rc = prompt_layers(b, tokens, table, prompt_workspace, static_cast<int32_t*>(b->workspace) + kBwCtl / 4, &x, s);
+  if (rc != LFM25_OK || (tokens_out == nullptr && hidden_out == nullptr)) return rc;
+  k_bx_last_rows<<<n_runs, kHidden / 8, 0, s>>>(p, table, x, hidden_out);
+  return tokens_out != nullptr ? launch_head(p, tokens_out, s) : check_launch("prompt pass rows");
 }
 
 int lfm25_batch_decode(const lfm25_batch* b, const int32_t* tokens_in, const int32_t* positions, int32_t n_steps,

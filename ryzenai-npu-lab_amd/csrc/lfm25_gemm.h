@@ -126,9 +126,9 @@ __device__ __forceinline__ void interleave() {
 }
 
 // acc += the block tile's product over `steps` K steps. The
-// descriptors cover whole rows (a lane offset at or past their size reads
-// zeros without touching memory; the step's offset is scalar and not
-// checked). Leaves no copy in flight.
+// descriptors cover the tile's rows inside the matrix (a lane offset past
+// them touches no memory, and what its row's products are is not used; the
+// step's offset is scalar and not checked). Leaves no copy in flight.
 template <typename S>
 __device__ __forceinline__ void product(Lds<S>& sh, const void* a_base, uint32_t a_bytes, const void* b_base,
                                         uint32_t b_bytes, const Copies<S>& c, int steps, Acc<S>& acc) {

@@ -29,6 +29,21 @@ int batch_decode_persistent(const lfm25_batch* b, void* region, int32_t* status,
                             const int32_t* positions, int32_t n_steps, int32_t* tokens_out, uint16_t* hidden_out,
                             hipStream_t s, bool prefix, int32_t* done);
 
+// The prompt pass's layers (lfm25_prompt.hip) behind lfm25_prompt_pass: the
+// rows of `runs`, run after run, with token ids tokens[row], through the
+// model; *x is then the last layer's output [rows][1024] in `ws`, which
+// holds prompt_bytes(rows) bytes.
+struct PromptRun {
+  int32_t sequence, position, count;
+};
+struct PromptRuns {
+  int32_t n;
+  PromptRun run[LFM25_BATCH_MAX_ROWS];
+};
+size_t prompt_bytes(int rows);
+int prompt_layers(const lfm25_batch* b, const int32_t* tokens, const PromptRuns& runs, void* ws, int32_t* status,
+                  const uint16_t** x, hipStream_t s);
+
 inline int check_launch(const char* what) {
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(LFM25_EDEVICE, "%s: %s", what, hipGetErrorString(e));

@@ -17,9 +17,8 @@ INT8 study ranks first, experiments/014_int8_lfm25.py); KV tiers are accepted fo
 but the GPU streams exactly the filled positions, so only the largest tier
 (the capacity) matters. `generate(prompt, n)` runs the prompt as prefill does
 and then the greedy tokens in one device call, with no host round trip per
-token. A prompt's tokens before the last go through matrix-core passes of up
-to 64 positions, as the reference's prefill sends its full PB batches
-through prefill_batch.
+token. A prompt's tokens before the last go through one matrix-core pass, as
+the reference's prefill sends its full PB batches through prefill_batch.
 """
 
 from __future__ import annotations
@@ -30,7 +29,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .batch import run_pass
+from .batch import PROMPT_ROWS, PromptWorkspace, run_pass, run_prompt
 from .bf16 import bf16_bits_to_f32
 from .weights import (HEAD_DIM, HIDDEN, KINDS, KV_HEADS, VOCAB, load_safetensors, pack_stream, pack_w8,
                       rope_table, synthetic_checkpoint)
@@ -38,7 +37,6 @@ from .weights import (HEAD_DIM, HIDDEN, KINDS, KV_HEADS, VOCAB, load_safetensors
 TIERS = (64, 256, 1024, 4096)
 MAX_CAPACITY = 4096
 PB = 4  # prompt tokens per batched call (experiments/lfm25_x8.py:79)
-PASS_ROWS = 64  # prompt positions per matrix-core pass (LFM25_BATCH_MAX_ROWS)
 CONV_LAYERS = KINDS.count("conv")
 ATT_LAYERS = KINDS.count("attention")
 
@@ -128,6 +126,7 @@ class X8Model:
                                     self.w8_table_scales.data_ptr())
         self._last_prompt_hidden = []
         self._batch = None
+        self._prompt_ws = PromptWorkspace(self.device)
         self._hidden_from_batch = False
         self.reset()
         torch.cuda.synchronize(self.device)
@@ -197,15 +196,17 @@ class X8Model:
                 raise ValueError(f"token id {t} outside the vocabulary")
 
     def _prefill_rows(self, tokens) -> None:
-        """Prompt positions without a selection, in matrix-core passes of up
-        to 64 rows on the decoder's own caches (lfm25_batch_pass), then the
-        position control word the decode continues from."""
+        """Prompt positions without a selection on the decoder's own caches
+        (one lfm25_prompt_pass, or below PROMPT_ROWS rows one
+        lfm25_batch_pass), then the position control word the decode continues from."""
         batch = self._batch_desc()
-        for start in range(0, len(tokens), PASS_ROWS):
-            chunk = tokens[start:start + PASS_ROWS]
-            rows = [(int(t), 0, self.position + i) for i, t in enumerate(chunk)]
+        if len(tokens) < PROMPT_ROWS:
+            rows = [(int(t), 0, self.position + i) for i, t in enumerate(tokens)]
             run_pass(batch, rows, False, None, None, self._stream())
-            self.position += len(chunk)
+        else:
+            ids = torch.tensor(tokens, dtype=torch.int32).to(self.device)
+            run_prompt(batch, self._prompt_ws, ids, [(0, self.position, len(tokens))], None, self._stream())
+        self.position += len(tokens)
         self.ctl[_lib.CTL_POSITION] = self.position
         status = int(self._batch_ws[:4].view(torch.int32).item())
         if status:
@@ -215,7 +216,7 @@ class X8Model:
     def _prompt(self, token_ids, n_gen: int) -> list[int]:
         """A prompt and n_gen greedy tokens, the way the reference's prefill
         runs a prompt (experiments/lfm25_x8_model.py:117-126): every token but
-        the last in matrix-core passes (when there are at least PB of them;
+        the last in a matrix-core pass (when there are at least PB of them;
         shorter bodies go token by token, one launch beating a pass), then the
         last token and the generated ones in one decode call."""
         tokens = [int(t) for t in token_ids]
@@ -253,8 +254,8 @@ class X8Model:
 
     def prefill(self, token_ids):
         """Process prompt tokens; the last one also selects the next token.
-        Returns the selected token id. The tokens before the last run in
-        matrix-core passes of up to 64 positions (at least PB of them)."""
+        Returns the selected token id. The tokens before the last run in one
+        matrix-core pass (at least PB of them)."""
         if len(token_ids) < 1:
             raise ValueError("prefill needs at least one token")
         return self._prompt(token_ids, 1)[0]
