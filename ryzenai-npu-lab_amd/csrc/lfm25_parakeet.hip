@@ -790,8 +790,10 @@ int enc_gemm_ln(const uint16_t* a, int lda, const uint16_t* bt, int m, int k, fl
 }
 
 // FP32 partial buffer of the encoder: split products (pick_splits) have at
-// most kCus blocks of the smallest tile.
-constexpr size_t kPartBytes = (size_t)tile::kCus * tile::S32x64::kTM * tile::S32x64::kTN * sizeof(float);
+// most kCus blocks of the smallest tile, 2 MB; the 32 MB that callers have
+// always been asked for stand.
+constexpr size_t kPartBytes = (size_t)32 << 20;
+static_assert((size_t)tile::kCus * tile::S32x64::kTM * tile::S32x64::kTN * sizeof(float) <= kPartBytes, "partials fit");
 
 // Workspace of the encoder for `rows` = batch * 128 frames (bytes).
 inline size_t pk_ws_bytes(int rows) {
