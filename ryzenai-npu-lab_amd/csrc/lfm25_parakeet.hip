@@ -789,15 +789,16 @@ int enc_gemm_ln(const uint16_t* a, int lda, const uint16_t* bt, int m, int k, fl
   return check_launch("parakeet gemm + layer norm");
 }
 
-// FP32 partial buffer of the encoder: split products (pick_splits) have at
-// most kCus blocks of the smallest tile, 2 MB; the 32 MB that callers have
-// always been asked for stand.
+// FP32 partial buffer of the encoder. Split products (pick_splits) have at
+// most kCus blocks of the smallest tile, 2 MB; callers are asked for what
+// they always were, 32 MB or a float per row and channel.
 constexpr size_t kPartBytes = (size_t)32 << 20;
 static_assert((size_t)tile::kCus * tile::S32x64::kTM * tile::S32x64::kTN * sizeof(float) <= kPartBytes, "partials fit");
+inline size_t pk_part_bytes(int rows) { return std::max(kPartBytes, (size_t)rows * kD * sizeof(float)); }
 
 // Workspace of the encoder for `rows` = batch * 128 frames (bytes).
 inline size_t pk_ws_bytes(int rows) {
-  return kPartBytes + (size_t)rows * 2 * (kD /*a*/ + kPkFfn /*big*/ + kD /*o*/);
+  return pk_part_bytes(rows) + (size_t)rows * 2 * (kD /*a*/ + kPkFfn /*big*/ + kD /*o*/);
 }
 
 }  // namespace
@@ -890,7 +891,7 @@ int lfm25_pk_encoder(const lfm25_pk_layer* layers, int32_t n_layers, uint16_t* x
   const int rows = batch * frames;
   char* ws = static_cast<char*>(workspace);
   float* part = reinterpret_cast<float*>(ws);
-  uint16_t* a = reinterpret_cast<uint16_t*>(ws + kPartBytes);
+  uint16_t* a = reinterpret_cast<uint16_t*>(ws + pk_part_bytes(rows));
   uint16_t* big = a + (size_t)rows * kD;
   uint16_t* o = big + (size_t)rows * kPkFfn;
   int rc = LFM25_OK;
