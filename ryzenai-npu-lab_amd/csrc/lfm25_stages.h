@@ -559,22 +559,4 @@ __device__ __forceinline__ void stage_head_scan(const uint16_t* h, const uint16_
   __syncthreads();
 }
 
-// Merge n candidates (one block); returns the winner in every thread of
-// wave 0 and writes it to *token when token != nullptr.
-__device__ __forceinline__ int pick_candidates(const Candidate* cand, int n) {
-  float bv = -INFINITY;
-  int bi = 0x7fffffff;
-  for (int i = lane_id(); i < n; i += kWave) {
-    const Candidate c = cand[i];
-    if (better(c.value, c.row, bv, bi)) { bv = c.value; bi = c.row; }
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(bv, o, kWave);
-    const int oi = __shfl_xor(bi, o, kWave);
-    if (better(ov, oi, bv, bi)) { bv = ov; bi = oi; }
-  }
-  return bi;
-}
-
 }  // namespace lfm25
