@@ -410,6 +410,41 @@ typedef struct lfm25_layer {
   const uint16_t* w2;             /* [1024 x 2560] */
 } lfm25_layer;
 
+/* One token through one layer by the reference's per-operation programs, a
+ * launch per dependent product. workspace: lfm25_layer_workspace_bytes()
+ * bytes, 16-byte aligned, contents ignored; calls sharing one must not
+ * overlap. A norm weight is a tile of 4,096 values, the first 1,024 used. */
+size_t lfm25_layer_workspace_bytes(void);
+
+/* A conv layer: packed_weights = [operator gamma tile | in_proj | out_proj |
+ * ffn gamma tile | w1 | w3 | w2]; next_state_and_weight = [next state (1024 x
+ * 3) | conv_weight (1024 x 3)] (state and conv_weight may lie in it).
+ * Replaces lfm25_single_program_block_kernel.py:32-284. */
+int lfm25_recurrent_block(const uint16_t* hidden, const uint16_t* state, const uint16_t* conv_weight,
+                          const uint16_t* packed_weights, uint16_t* next_state_and_weight, uint16_t* block_output,
+                          void* workspace, lfm25_stream_t stream);
+
+/* qkv_output = [q | k | v] (2048) of RMSNorm(hidden), q and k per head through
+ * QK norm and RoPE, then hidden (1024) when include_hidden; packed = [gamma
+ * tile | q | k | v], aux = [q_gamma (64) | k_gamma (64) | cos (64) | sin (64)].
+ * Replaces lfm25_attention_prefix_kernel.py:22-140. */
+int lfm25_attention_prefix(const uint16_t* hidden, const uint16_t* packed_gamma_and_weight, const uint16_t* aux,
+                           uint16_t* qkv_output, int32_t include_hidden, lfm25_stream_t stream);
+
+/* lfm25_attention_context into packed_tail_input[1024 ..], the hidden part of
+ * qkv_and_hidden into packed_tail_input[0 .. 1024), and
+ * lfm25_attention_append_cache into next_cache, with 1 <= past_length < 4096.
+ * Replaces lfm25_attention_context_cache_kernel.py:16-106. */
+int lfm25_attention_context_cache(const uint16_t* qkv_and_hidden, const uint16_t* past_cache,
+                                  uint16_t* packed_tail_input, uint16_t* next_cache, int32_t past_length,
+                                  void* workspace, lfm25_stream_t stream);
+
+/* block_output = h + w2 . (silu(w1 . n) * (w3 . n)), h = hidden + o . context, n
+ * = RMSNorm(h); packed_weights = [o | ffn gamma tile | w1 | w3 | w2]. Replaces
+ * lfm25_attention_tail_kernel.py:29-208. */
+int lfm25_attention_tail(const uint16_t* packed_hidden_and_context, const uint16_t* packed_weights,
+                         uint16_t* block_output, void* workspace, lfm25_stream_t stream);
+
 /* hidden_out[1024] = the layer applied to hidden_in[1024] at `position`
  * (attention: the token's key / value row is appended there and positions
  * [0, position] are attended; conv: conv_state_out gets the shifted state).

@@ -92,6 +92,11 @@ SIGNATURES = {
     "lfm25_attention_norm_rope": (ctypes.c_int, [_p, _p, _p]),
     "lfm25_attention_context": (ctypes.c_int, [_p, _p, _p, _i32, _p]),
     "lfm25_attention_append_cache": (ctypes.c_int, [_p, _p, _p, _i32, _p]),
+    "lfm25_layer_workspace_bytes": (_size, []),
+    "lfm25_recurrent_block": (ctypes.c_int, [_p, _p, _p, _p, _p, _p, _p, _p]),
+    "lfm25_attention_prefix": (ctypes.c_int, [_p, _p, _p, _p, _i32, _p]),
+    "lfm25_attention_context_cache": (ctypes.c_int, [_p, _p, _p, _p, _i32, _p, _p]),
+    "lfm25_attention_tail": (ctypes.c_int, [_p, _p, _p, _p, _p]),
     "lfm25_attention_first_context": (ctypes.c_int, [_p, _p, _p, _p]),
     "lfm25_attention_fixed": (ctypes.c_int, [_p, _p, _p, _p, _i32, _i32, _p, _p]),
     "lfm25_pack_block_input": (ctypes.c_int, [_p, _p, _p, _p]),

@@ -12,8 +12,6 @@ without waiting; NPU-only knobs such as n_cores are validated and ignored.
 
 from __future__ import annotations
 
-import ctypes
-
 import torch
 
 from . import _lib
@@ -150,55 +148,31 @@ def conv_gate_packed_state(projection, state_and_weight, output, next_state_and_
               _bf(next_state_and_weight, "next_state_and_weight", 6 * HIDDEN), _stream())
 
 
+# [operator gamma tile | in_proj | out_proj | ffn gamma tile | w1 | w3 | w2]
+_CONV_LAYER = 2 * GAMMA_TILE + (3 * HIDDEN + HIDDEN + 2 * FFN) * HIDDEN + HIDDEN * FFN
+
+
 def _layer_workspace(device) -> torch.Tensor:
-    """A zeroed lfm25_decode_layer workspace for one call (its exchange epochs
-    start from zero, so concurrent calls never share one)."""
-    return torch.zeros(int(_lib.load().lfm25_decoder_workspace_bytes()), dtype=torch.uint8, device=device)
+    """Scratch memory for one call of the layer programs (so concurrent calls
+    never share one; the caching allocator hands the same memory out again)."""
+    return torch.empty(_lib.load().lfm25_layer_workspace_bytes(), dtype=torch.uint8, device=device)
 
 
 def recurrent_block(packed_hidden_and_state, packed_weights, next_state_and_weight,
                     block_output) -> None:
-    """One conv decoder layer in one launch (lfm25_decode_layer).
+    """One conv decoder layer (lfm25_recurrent_block).
     Reference: lfm25_single_program_block_kernel.py:32-284.
     packed_hidden_and_state = [hidden (1024) | pad to 6144 | state (1024 x 3) |
     conv w (1024 x 3)]; packed_weights = [operator gamma tile | in_proj |
     out_proj | ffn gamma tile | w1 | w3 | w2]; next_state_and_weight =
     [next state (1024 x 3) | conv w (1024 x 3)]."""
     hp = _bf(packed_hidden_and_state, "packed_hidden_and_state", 2 * 6144)
-    n_w = 2 * GAMMA_TILE + (3 * HIDDEN + HIDDEN + 2 * FFN) * HIDDEN + HIDDEN * FFN
-    wp = _bf(packed_weights, "packed_weights", n_w)
+    wp = _bf(packed_weights, "packed_weights", _CONV_LAYER)
     nxt = _bf(next_state_and_weight, "next_state_and_weight", 6144)
     out = _bf(block_output, "block_output", HIDDEN)
-    at = lambda elems: wp + 2 * elems  # noqa: E731  (byte address of element `elems`)
-    o_out = GAMMA_TILE + 3 * HIDDEN * HIDDEN
-    o_ffn = o_out + HIDDEN * HIDDEN
-    o_w1 = o_ffn + GAMMA_TILE
-    layer = _lib.Layer(kind=_lib.LAYER_CONV, op_norm=wp, mixer=at(GAMMA_TILE),
-                       conv_weight=hp + 2 * (6144 + 3 * HIDDEN), conv_state_in=hp + 2 * 6144,
-                       conv_state_out=nxt, out=at(o_out), ffn_norm=at(o_ffn), w1=at(o_w1),
-                       w3=at(o_w1 + FFN * HIDDEN), w2=at(o_w1 + 2 * FFN * HIDDEN))
     ws = _layer_workspace(block_output.device)
-    _lib.call("lfm25_decode_layer", ctypes.byref(layer), hp, out, 0, ws.data_ptr(), _stream())
-    next_state_and_weight[3 * HIDDEN:].copy_(packed_hidden_and_state[6144 + 3 * HIDDEN:])
-
-
-def _mlp_tail(residual, projection_input, weights, block_output) -> None:
-    """[out (1024 x 1024) | ffn gamma tile | w1 | w3 | w2] applied as
-    h = residual + out.x; block_output = h + w2.(silu(w1.n) * w3.n), n = norm(h)."""
-    dev = block_output.device
-    proj = torch.empty(HIDDEN, dtype=torch.bfloat16, device=dev)
-    bf16_bf16_gemv(weights[:HIDDEN * HIDDEN], projection_input, proj, M=HIDDEN, K=HIDDEN)
-    h = torch.empty(HIDDEN, dtype=torch.bfloat16, device=dev)
-    bf16_add(residual, proj, h, N=HIDDEN)
-    off = HIDDEN * HIDDEN
-    up = torch.empty(2 * FFN, dtype=torch.bfloat16, device=dev)
-    norm_bf16_gemv(h, weights[off:off + GAMMA_TILE + 2 * FFN * HIDDEN], up, M=2 * FFN, K=HIDDEN)
-    gate = torch.empty(FFN, dtype=torch.bfloat16, device=dev)
-    silu_gate(up[:FFN], up[FFN:], gate, N=FFN)
-    off += GAMMA_TILE + 2 * FFN * HIDDEN
-    down = torch.empty(HIDDEN, dtype=torch.bfloat16, device=dev)
-    bf16_bf16_gemv(weights[off:off + HIDDEN * FFN], gate, down, M=HIDDEN, K=FFN)
-    bf16_add(h, down, block_output, N=HIDDEN)
+    _lib.call("lfm25_recurrent_block", hp, hp + 2 * 6144, hp + 2 * (6144 + 3 * HIDDEN), wp, nxt, out, ws.data_ptr(),
+              _stream())
 
 
 # ---------------------------------------------------------------- attention
@@ -211,16 +185,11 @@ def attention_prefix(hidden, packed_weights, qkv_output, *, include_hidden: bool
     Reference: lfm25_attention_prefix_kernel.py:22-140; packed_weights =
     [gamma tile | q | k | v | aux tile = q_gamma (64) | k_gamma (64) | cos (64) |
     sin (64)]."""
-    n_w = 2 * GAMMA_TILE + _QKV * HIDDEN
-    _bf(packed_weights, "packed_weights", n_w)
-    _bf(qkv_output, "qkv_output", _QKV + (HIDDEN if include_hidden else 0))
-    norm_bf16_gemv(hidden, packed_weights[:GAMMA_TILE + _QKV * HIDDEN], qkv_output[:_QKV],
-                   M=_QKV, K=HIDDEN)
-    aux = packed_weights[GAMMA_TILE + _QKV * HIDDEN:GAMMA_TILE + _QKV * HIDDEN + 256]
-    _lib.call("lfm25_attention_norm_rope", _bf(qkv_output, "qkv_output"), aux.data_ptr(),
+    h = _bf(hidden, "hidden", HIDDEN)
+    w = _bf(packed_weights, "packed_weights", 2 * GAMMA_TILE + _QKV * HIDDEN)
+    out = _bf(qkv_output, "qkv_output", _QKV + (HIDDEN if include_hidden else 0))
+    _lib.call("lfm25_attention_prefix", h, w, w + 2 * (GAMMA_TILE + _QKV * HIDDEN), out, 1 if include_hidden else 0,
               _stream())
-    if include_hidden:
-        qkv_output[_QKV:].copy_(hidden)
 
 
 def _past_length(cache, name: str) -> int:
@@ -253,25 +222,28 @@ def attention_context_cache(qkv_and_hidden, past_cache, packed_tail_input, next_
     packed_tail_input = [hidden (1024) | context (1024)]."""
     if not 1 <= past_length < 4096:
         raise ValueError("past_length must be in [1, 4096)")
-    _bf(qkv_and_hidden, "qkv_and_hidden", _QKV + HIDDEN)
-    _bf(past_cache, "past_cache", 2 * 8 * past_length * 64)
-    _bf(packed_tail_input, "packed_tail_input", 2 * HIDDEN)
-    _bf(next_cache, "next_cache", 2 * 8 * (past_length + 1) * 64)
-    attention_context(qkv_and_hidden[:_QKV], past_cache, packed_tail_input[HIDDEN:])
-    append_attention_cache(qkv_and_hidden[:_QKV], past_cache, next_cache)
-    packed_tail_input[:HIDDEN].copy_(qkv_and_hidden[_QKV:])
+    qkv = _bf(qkv_and_hidden, "qkv_and_hidden", _QKV + HIDDEN)
+    past = _bf(past_cache, "past_cache", 2 * 8 * past_length * 64)
+    tail = _bf(packed_tail_input, "packed_tail_input", 2 * HIDDEN)
+    nxt = _bf(next_cache, "next_cache", 2 * 8 * (past_length + 1) * 64)
+    if (qkv | nxt) & 15:  # the one-pass form moves whole 16-byte pieces
+        attention_context(qkv_and_hidden[:_QKV], past_cache, packed_tail_input[HIDDEN:])
+        append_attention_cache(qkv_and_hidden[:_QKV], past_cache, next_cache)
+        packed_tail_input[:HIDDEN].copy_(qkv_and_hidden[_QKV:])
+        return
+    ws = _layer_workspace(next_cache.device)
+    _lib.call("lfm25_attention_context_cache", qkv, past, tail, nxt, past_length, ws.data_ptr(), _stream())
 
 
 def attention_tail(packed_hidden_and_context, packed_weights, block_output) -> None:
     """o_proj + residual + SwiGLU MLP + residual.
     Reference: lfm25_attention_tail_kernel.py:29-208; packed_weights = [o |
     ffn gamma tile | w1 | w3 | w2]."""
-    _bf(packed_hidden_and_context, "packed_hidden_and_context", 2 * HIDDEN)
-    n_w = HIDDEN * HIDDEN + GAMMA_TILE + 3 * FFN * HIDDEN
-    _bf(packed_weights, "packed_weights", n_w)
-    _bf(block_output, "block_output", HIDDEN)
-    _mlp_tail(packed_hidden_and_context[:HIDDEN], packed_hidden_and_context[HIDDEN:],
-              packed_weights, block_output)
+    x = _bf(packed_hidden_and_context, "packed_hidden_and_context", 2 * HIDDEN)
+    w = _bf(packed_weights, "packed_weights", HIDDEN * HIDDEN + GAMMA_TILE + 3 * FFN * HIDDEN)
+    out = _bf(block_output, "block_output", HIDDEN)
+    ws = _layer_workspace(block_output.device)
+    _lib.call("lfm25_attention_tail", x, w, out, ws.data_ptr(), _stream())
 
 
 # ---------------------------------------------------------------- head / embedding
@@ -400,24 +372,14 @@ def norm_proj_conv(packed_hidden_and_state, packed_gamma_and_projection_weight, 
 
 def _pair_layer(hiddens, state_in, conv_w, packed_weights, next_state_and_weight, block_output) -> None:
     """Two consecutive positions through one conv layer: the second starts
-    from the state the first left (lfm25_decode_layer twice, in place)."""
-    n_w = 2 * GAMMA_TILE + (3 * HIDDEN + HIDDEN + 2 * FFN) * HIDDEN + HIDDEN * FFN
-    wp = _bf(packed_weights, "packed_weights", n_w)
+    from the state the first left (lfm25_recurrent_block twice, in place)."""
+    wp = _bf(packed_weights, "packed_weights", _CONV_LAYER)
     nxt = _bf(next_state_and_weight, "next_state_and_weight", 6144)
-    _bf(block_output, "block_output", 2 * HIDDEN)
-    at = lambda elems: wp + 2 * elems  # noqa: E731
-    o_out = GAMMA_TILE + 3 * HIDDEN * HIDDEN
-    o_ffn = o_out + HIDDEN * HIDDEN
-    o_w1 = o_ffn + GAMMA_TILE
+    out = _bf(block_output, "block_output", 2 * HIDDEN)
     ws = _layer_workspace(block_output.device)
     for i, h in enumerate(hiddens):
-        layer = _lib.Layer(kind=_lib.LAYER_CONV, op_norm=wp, mixer=at(GAMMA_TILE), conv_weight=conv_w.data_ptr(),
-                           conv_state_in=state_in.data_ptr() if i == 0 else nxt, conv_state_out=nxt,
-                           out=at(o_out), ffn_norm=at(o_ffn), w1=at(o_w1), w3=at(o_w1 + FFN * HIDDEN),
-                           w2=at(o_w1 + 2 * FFN * HIDDEN))
-        _lib.call("lfm25_decode_layer", ctypes.byref(layer), h.data_ptr(),
-                  block_output[i * HIDDEN:(i + 1) * HIDDEN].data_ptr(), 0, ws.data_ptr(), _stream())
-    next_state_and_weight[3 * HIDDEN:].copy_(conv_w)
+        _lib.call("lfm25_recurrent_block", h.data_ptr(), state_in.data_ptr() if i == 0 else nxt, conv_w.data_ptr(), wp,
+                  nxt, out + 2 * i * HIDDEN, ws.data_ptr(), _stream())
 
 
 def recurrent_pair_block(packed_hidden_and_state, packed_weights, next_state_and_weight, block_output) -> None:
@@ -447,16 +409,12 @@ def attention_prefix_pair(hidden_pair, packed_weights_and_aux0, aux1, qkv_pair) 
     (3072) | the same of the second]; aux0 (the first position's QK-norm and
     RoPE tile) ends packed_weights_and_aux0, aux1 is the second's.
     Reference: lfm25_prefill_pair_attention_prefix_kernel.py:23."""
-    _bf(hidden_pair, "hidden_pair", 2 * HIDDEN)
-    _bf(aux1, "aux1", GAMMA_TILE)
-    _bf(qkv_pair, "qkv_pair", 2 * (_QKV + HIDDEN))
-    w = packed_weights_and_aux0
-    _bf(w, "packed_weights_and_aux0", 2 * GAMMA_TILE + _QKV * HIDDEN)
-    attention_prefix(hidden_pair[:HIDDEN], w, qkv_pair[:_QKV + HIDDEN], include_hidden=True)
-    second = qkv_pair[_QKV + HIDDEN:]
-    norm_bf16_gemv(hidden_pair[HIDDEN:], w[:GAMMA_TILE + _QKV * HIDDEN], second[:_QKV], M=_QKV, K=HIDDEN)
-    _lib.call("lfm25_attention_norm_rope", second.data_ptr(), aux1.data_ptr(), _stream())
-    second[_QKV:].copy_(hidden_pair[HIDDEN:])
+    h = _bf(hidden_pair, "hidden_pair", 2 * HIDDEN)
+    second = _bf(aux1, "aux1", GAMMA_TILE)
+    out = _bf(qkv_pair, "qkv_pair", 2 * (_QKV + HIDDEN))
+    w = _bf(packed_weights_and_aux0, "packed_weights_and_aux0", 2 * GAMMA_TILE + _QKV * HIDDEN)
+    for i, aux in enumerate((w + 2 * (GAMMA_TILE + _QKV * HIDDEN), second)):
+        _lib.call("lfm25_attention_prefix", h + 2 * i * HIDDEN, w, aux, out + 2 * i * (_QKV + HIDDEN), 1, _stream())
 
 
 def attention_tail_pair(packed_hidden_and_context, packed_weights, block_output) -> None:
