@@ -219,13 +219,21 @@ __device__ __forceinline__ void each_row(const Acc<S>& acc, int m0, int n0, int 
   }
 }
 
+// Two floats as a BF16 pair, low first: one v_cvt_pk_bf16_f32 (two separate
+// conversions become two of them and two more to join the halves).
+__device__ __forceinline__ uint32_t pack_pair(float lo, float hi) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
+}
+
 // kN consecutive values as BF16 pairs; p is 8-byte aligned, 16-byte where
 // `wide` (16-byte stores need it).
 template <int kN>
 __device__ __forceinline__ void store_bf16(uint16_t* p, const float (&v)[kN], bool wide) {
   uint32_t o[kN / 2];
 #pragma unroll
-  for (int i = 0; i < kN / 2; ++i) o[i] = (uint32_t)f32_to_bf16(v[2 * i]) | ((uint32_t)f32_to_bf16(v[2 * i + 1]) << 16);
+  for (int i = 0; i < kN / 2; ++i) o[i] = pack_pair(v[2 * i], v[2 * i + 1]);
   if constexpr (kN % 8 == 0) {
     if (wide) {
 #pragma unroll

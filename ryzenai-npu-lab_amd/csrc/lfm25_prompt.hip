@@ -59,9 +59,7 @@ __device__ __forceinline__ size_t pp_kv_base(const Prompt& p, int seq, int att, 
   return ((size_t)(seq * LFM25_ATTN_LAYERS + att) * kKvHeads + g) * p.capacity * kHeadDim;
 }
 
-__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  return (uint32_t)f32_to_bf16(lo) | ((uint32_t)f32_to_bf16(hi) << 16);
-}
+using tile::pack_pair;
 
 // ------------------------------------------------------------------ norms
 
@@ -72,8 +70,8 @@ __device__ __forceinline__ void store_lane_vec(uint16_t* row, const LaneVec<kHid
 #pragma unroll
   for (int c = 0; c < LaneVec<kHidden>::kChunks; ++c)
     *reinterpret_cast<uint4*>(row + c * 512 + lane_id() * 8) =
-        uint4{pack2(v.v[8 * c], v.v[8 * c + 1]), pack2(v.v[8 * c + 2], v.v[8 * c + 3]),
-              pack2(v.v[8 * c + 4], v.v[8 * c + 5]), pack2(v.v[8 * c + 6], v.v[8 * c + 7])};
+        uint4{pack_pair(v.v[8 * c], v.v[8 * c + 1]), pack_pair(v.v[8 * c + 2], v.v[8 * c + 3]),
+              pack_pair(v.v[8 * c + 4], v.v[8 * c + 5]), pack_pair(v.v[8 * c + 6], v.v[8 * c + 7])};
 }
 
 // Row m of x = the embedding row of its token (ids outside the table are
@@ -160,7 +158,7 @@ __global__ void __launch_bounds__(S::kThreads, 2) k_pp_gemm(const PpGemm g) {
       if constexpr (kHalf >= 4) {
         tile::store_bf16<kHalf>(c, f, true);
       } else {
-        *reinterpret_cast<uint32_t*>(c) = pack2(f[0], f[1]);
+        *reinterpret_cast<uint32_t*>(c) = pack_pair(f[0], f[1]);
       }
     } else {
       uint16_t* c = g.c + (size_t)m * g.ldc + n;
@@ -322,9 +320,8 @@ __device__ __forceinline__ float sum_groups(float v) {
   return __uint_as_float(c[0]) + __uint_as_float(c[1]);
 }
 
-// Causal attention of kQ query positions of one run (blockIdx.x), KV head
-// blockIdx.y: the two query heads' columns share every key and value tile.
-// The eager form's numbers (s_j = bf16(q . k_j) * 0.125; p_j = bf16(e^(s_j - m)
+// Causal attention of kQ query positions of one run and one KV head: the two
+// query heads' columns share every key and value tile. The eager form's numbers (s_j = bf16(q . k_j) * 0.125; p_j = bf16(e^(s_j - m)
 // / z); ctx = bf16(sum_j p_j v_j)) need m and z before the first p, so the
 // keys are passed twice: once for m and z, once for the context. A wave owns
 // 16 columns (one head, 16 positions); keys are the products' rows, so a lane
@@ -375,8 +372,17 @@ __global__ void __launch_bounds__(kQ * 8) k_pp_attention(Prompt p, PromptRuns ru
 #if defined(__HIP_DEVICE_COMPILE__)  // (the host pass has no LDS address space)
   constexpr int kWaves = kQ / 8, kCopies = 8 / kWaves;  // copy instructions per wave and 64-row tile
   __shared__ AttLds sh;
-  // the run and its tile; a run's last (longest) tiles come first
-  int r = 0, first = 0, tile_at = blockIdx.x;
+  // This block's KV head and query tile. Tiles cost by their position, and up
+  // to about two blocks land on a CU, block i and block i + 256: the first
+  // half of the blocks takes the tiles from the longest down, the second half
+  // the rest from the shortest up, so that a CU's two add up to the same
+  // (3,900 rows: 151 -> 113 us; with the heads apart in the grid a CU could
+  // get two of the longest). Consecutive blocks are the eight heads, so an
+  // XCD reads one head's keys and values at a time.
+  const int half = gridDim.x / (2 * kKvHeads) * kKvHeads, i = blockIdx.x;
+  const int rank = i < half ? i : (int)gridDim.x - 1 - (i - half);
+  const int g = rank % kKvHeads;
+  int r = 0, first = 0, tile_at = rank / kKvHeads;
   while (true) {
     const int tiles = (runs.run[r].count + kQ - 1) / kQ;
     if (tile_at < tiles) {
@@ -387,7 +393,7 @@ __global__ void __launch_bounds__(kQ * 8) k_pp_attention(Prompt p, PromptRuns ru
     first += runs.run[r++].count;
   }
   const int count = runs.run[r].count, pos0 = runs.run[r].position, seq = runs.run[r].sequence;
-  const int g = blockIdx.y, w = wave_id(), l = lane_id();
+  const int w = wave_id(), l = lane_id();
   const int q0 = tile_at * kQ;                              // the block's first query within the run
   const int end = pos0 + min(q0 + kQ, count);               // cached positions any of its queries sees
   const int tiles = (end + kKeys - 1) / kKeys;
@@ -447,7 +453,7 @@ __global__ void __launch_bounds__(kQ * 8) k_pp_attention(Prompt p, PromptRuns ru
     for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
       for (int e = 0; e < 4; e += 2) {
-        const uint32_t b = pack2(s[kt][e], s[kt][e + 1]);
+        const uint32_t b = pack_pair(s[kt][e], s[kt][e + 1]);
         s[kt][e] = lo_f32(b);
         s[kt][e + 1] = hi_f32(b);
       }
@@ -514,7 +520,7 @@ __global__ void __launch_bounds__(kQ * 8) k_pp_attention(Prompt p, PromptRuns ru
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const f32x4& sk = s[2 * c + i / 2];
-        pw[i] = pack2(__builtin_amdgcn_exp2f(fmaf(sk[2 * (i % 2)], kC, -mc)) * rz,
+        pw[i] = pack_pair(__builtin_amdgcn_exp2f(fmaf(sk[2 * (i % 2)], kC, -mc)) * rz,
                       __builtin_amdgcn_exp2f(fmaf(sk[2 * (i % 2) + 1], kC, -mc)) * rz);
       }
       const bf16x8 pf = __builtin_bit_cast(bf16x8, uint4{pw[0], pw[1], pw[2], pw[3]});
@@ -534,7 +540,7 @@ __global__ void __launch_bounds__(kQ * 8) k_pp_attention(Prompt p, PromptRuns ru
   uint16_t* dst = p.y + (size_t)row * kHidden + (2 * g + w % 2) * kHeadDim + 4 * (l >> 4);
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt)
-    *reinterpret_cast<uint2*>(dst + 16 * dt) = uint2{pack2(o[dt][0], o[dt][1]), pack2(o[dt][2], o[dt][3])};
+    *reinterpret_cast<uint2*>(dst + 16 * dt) = uint2{pack_pair(o[dt][0], o[dt][1]), pack_pair(o[dt][2], o[dt][3])};
 #endif
 }
 
@@ -542,7 +548,7 @@ template <int kQ>
 void launch_attention(const Prompt& p, const PromptRuns& runs, int att, hipStream_t s) {
   int tiles = 0;
   for (int r = 0; r < runs.n; ++r) tiles += (runs.run[r].count + kQ - 1) / kQ;
-  k_pp_attention<kQ><<<dim3(tiles, kKvHeads), kQ * 8, 0, s>>>(p, runs, att);
+  k_pp_attention<kQ><<<tiles * kKvHeads, kQ * 8, 0, s>>>(p, runs, att);
 }
 
 }  // namespace
