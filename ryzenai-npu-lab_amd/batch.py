@@ -77,12 +77,13 @@ class PromptWorkspace:
 
 
 def run_prompt(desc: _lib.Batch, workspace: PromptWorkspace, tokens: torch.Tensor, runs: list[tuple[int, int, int]],
-               tokens_out: torch.Tensor | None, stream: int) -> None:
+               tokens_out: torch.Tensor | None, stream: int, hidden_out: torch.Tensor | None = None) -> None:
     """One lfm25_prompt_pass over `runs` = [(sequence, position, count), ...]
     of the device token ids `tokens`."""
     table = np.ascontiguousarray(np.asarray(runs, dtype=np.int32).reshape(-1, 3))
     _lib.call("lfm25_prompt_pass", ctypes.byref(desc), tokens.data_ptr(), table.ctypes.data, len(table),
-              tokens_out.data_ptr() if tokens_out is not None else None, None,
+              tokens_out.data_ptr() if tokens_out is not None else None,
+              hidden_out.data_ptr() if hidden_out is not None else None,
               workspace.pointer(int(table[:, 2].sum())), stream)
 
 

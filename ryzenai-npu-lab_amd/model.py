@@ -17,8 +17,8 @@ INT8 study ranks first, experiments/014_int8_lfm25.py); KV tiers are accepted fo
 but the GPU streams exactly the filled positions, so only the largest tier
 (the capacity) matters. `generate(prompt, n)` runs the prompt as prefill does
 and then the greedy tokens in one device call, with no host round trip per
-token. A prompt's tokens before the last go through one matrix-core pass, as
-the reference's prefill sends its full PB batches through prefill_batch.
+token. A prompt goes through one matrix-core pass, as the reference's prefill
+sends its full PB batches through prefill_batch.
 """
 
 from __future__ import annotations
@@ -127,7 +127,8 @@ class X8Model:
         self._last_prompt_hidden = []
         self._batch = None
         self._prompt_ws = PromptWorkspace(self.device)
-        self._hidden_from_batch = False
+        self._selected = torch.zeros(_lib.BATCH_MAX_ROWS, dtype=torch.int32, device=self.device)
+        self._hidden_from = None  # a pass's last row, when it ran last
         self.reset()
         torch.cuda.synchronize(self.device)
         log(f"weights ready in {time.perf_counter() - t0:.1f} s")
@@ -139,7 +140,7 @@ class X8Model:
 
     def reset(self):
         self.position = 0
-        self._hidden_from_batch = False
+        self._hidden_from = None  # a pass's last row, when it ran last
         _lib.call("lfm25_decoder_reset", self._desc, self._stream())
 
     def _run(self, tokens, n_gen: int) -> list[int]:
@@ -165,7 +166,7 @@ class X8Model:
         if status:
             raise RuntimeError(f"decode run ended with status 0x{status:x}")
         self.position += steps
-        self._hidden_from_batch = False
+        self._hidden_from = None  # a pass's last row, when it ran last
         return [int(t) for t in out]
 
     # ------------------------------------------------------------ reference API
@@ -195,37 +196,46 @@ class X8Model:
             if not 0 <= int(t) < self.vocab:
                 raise ValueError(f"token id {t} outside the vocabulary")
 
-    def _prefill_rows(self, tokens) -> None:
-        """Prompt positions without a selection on the decoder's own caches
-        (one lfm25_prompt_pass, or below PROMPT_ROWS rows one
-        lfm25_batch_pass), then the position control word the decode continues from."""
+    def _prompt(self, token_ids, n_gen: int) -> list[int]:
+        """A prompt and n_gen greedy tokens, the way the reference's prefill
+        runs a prompt (experiments/lfm25_x8_model.py:117-126): the prompt and
+        its selection in one matrix-core pass (lfm25_prompt_pass, below
+        PROMPT_ROWS tokens lfm25_batch_pass; at most PB tokens go token by
+        token, one launch beating a pass), then the other tokens in one
+        decode call, which reads the first on the device."""
+        tokens = [int(t) for t in token_ids]
+        self._check_tokens(tokens, len(tokens) + max(n_gen - 1, 0))
+        rows = len(tokens)
+        if rows <= PB or not self.batched_prefill:
+            return self._run(tokens, n_gen)
         batch = self._batch_desc()
-        if len(tokens) < PROMPT_ROWS:
-            rows = [(int(t), 0, self.position + i) for i, t in enumerate(tokens)]
-            run_pass(batch, rows, False, None, None, self._stream())
+        if rows < PROMPT_ROWS:
+            hidden = torch.empty(rows * HIDDEN, dtype=torch.bfloat16, device=self.device)
+            run_pass(batch, [(t, 0, self.position + i) for i, t in enumerate(tokens)], True, self._selected, hidden,
+                     self._stream())
+            first = self._selected[rows - 1:rows]
         else:
+            hidden = torch.empty(HIDDEN, dtype=torch.bfloat16, device=self.device)
             ids = torch.tensor(tokens, dtype=torch.int32).to(self.device)
-            run_prompt(batch, self._prompt_ws, ids, [(0, self.position, len(tokens))], None, self._stream())
-        self.position += len(tokens)
+            run_prompt(batch, self._prompt_ws, ids, [(0, self.position, rows)], self._selected, self._stream(), hidden)
+            first = self._selected[:1]
+        self.position += rows
         self.ctl[_lib.CTL_POSITION] = self.position
+        self.ctl[_lib.CTL_TOKEN:_lib.CTL_TOKEN + 1].copy_(first)  # what a decode without tokens_in continues from
+        if n_gen > 1:
+            _lib.call("lfm25_decode", self._desc, first.data_ptr(), 1, n_gen - 1, self._tokens_out.data_ptr(),
+                      self.exec, self._stream())
+        out = first.cpu().tolist() + (self._tokens_out[:n_gen - 1].cpu().tolist() if n_gen > 1 else [])
         status = int(self._batch_ws[:4].view(torch.int32).item())
         if status:
             raise RuntimeError(f"batched pass ended with status 0x{status:x}")
-        self._hidden_from_batch = False
-
-    def _prompt(self, token_ids, n_gen: int) -> list[int]:
-        """A prompt and n_gen greedy tokens, the way the reference's prefill
-        runs a prompt (experiments/lfm25_x8_model.py:117-126): every token but
-        the last in a matrix-core pass (when there are at least PB of them;
-        shorter bodies go token by token, one launch beating a pass), then the
-        last token and the generated ones in one decode call."""
-        tokens = [int(t) for t in token_ids]
-        self._check_tokens(tokens, len(tokens) + max(n_gen - 1, 0))
-        body = tokens[:-1]
-        if len(body) < PB or not self.batched_prefill:
-            return self._run(tokens, n_gen)
-        self._prefill_rows(body)
-        return self._run(tokens[-1:], n_gen)
+        if n_gen > 1:
+            status = int(self.ctl[_lib.CTL_STATUS].item())
+            if status:
+                raise RuntimeError(f"decode run ended with status 0x{status:x}")
+            self.position += n_gen - 1
+        self._hidden_from = None if n_gen > 1 else hidden[-HIDDEN:]
+        return [int(t) for t in out]
 
     def prefill_batch(self, token_ids):
         """PB prompt positions in one batched pass, no token selection (the
@@ -250,12 +260,12 @@ class X8Model:
         self.ctl[_lib.CTL_POSITION] = self.position
         hidden = _to_f32(h).reshape(PB, HIDDEN)
         self._last_prompt_hidden = [hidden[t] for t in range(PB)]
-        self._hidden_from_batch = True
+        self._hidden_from = h[-HIDDEN:]
 
     def prefill(self, token_ids):
         """Process prompt tokens; the last one also selects the next token.
-        Returns the selected token id. The tokens before the last run in one
-        matrix-core pass (at least PB of them)."""
+        Returns the selected token id. The prompt runs in one matrix-core pass
+        (more than PB tokens)."""
         if len(token_ids) < 1:
             raise ValueError("prefill needs at least one token")
         return self._prompt(token_ids, 1)[0]
@@ -271,8 +281,8 @@ class X8Model:
 
     def hidden(self) -> np.ndarray:
         """Pre-final-norm output of the last layer for the latest position."""
-        if self._hidden_from_batch:
-            return self._last_prompt_hidden[-1]
+        if self._hidden_from is not None:
+            return _to_f32(self._hidden_from)
         words = self._h_words.cpu().numpy().view(np.uint32)
         return bf16_bits_to_f32((words & 0xFFFF).astype(np.uint16))
 
