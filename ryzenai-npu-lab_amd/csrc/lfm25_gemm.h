@@ -326,7 +326,7 @@ struct Tiles {
   bool rects;
   __host__ __device__ int rect_m() const { return (m + 1) / 2; }
   __host__ __device__ int rect_n() const { return (n + 3) / 4; }
-  int blocks() const { return rects ? 8 * rect_m() * rect_n() : m * n; }
+  __host__ __device__ int blocks() const { return rects ? 8 * rect_m() * rect_n() : m * n; }
   // False for a block past the tiles (a rectangle that sticks out).
   __device__ bool of(int block, int& tm, int& tn) const {
     if (!rects) {
@@ -344,6 +344,20 @@ template <typename S>
 inline Tiles tiles_of(int m, int n, int64_t a_bytes) {
   const int tm = (m + S::kTM - 1) / S::kTM, tn = n / S::kTN;
   return Tiles{tm, tn, a_bytes > (4 << 20) && tm >= 8 && tn >= 4};
+}
+
+// The tile width of an m-row product whose weights' way from HBM bounds it
+// (their rows go to the XCDs in groups of it), or 0: not where the products
+// are long enough to hide it (1,024 rows and more), nor where the tiles are
+// dealt out in another order.
+inline int ahead_group(int m, int n, int splits, int64_t a_bytes) {
+  if (m > 1024) return 0;
+  int group = 0;
+  with_shape(m, n, splits, [&](auto shape) {
+    const Tiles t = tiles_of<decltype(shape)>(m, n, a_bytes);
+    group = t.rects || t.n % 8 != 0 ? 0 : decltype(shape)::kTN;
+  });
+  return group;
 }
 
 }  // namespace tile

@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "lfm25_host.h"
+#include "lfm25_ahead.h"
 #include "lfm25_device.h"
 #include "lfm25_gemm.h"
 
@@ -79,6 +80,7 @@ struct PkGemm {
   int lda, ldb, ldc, M, N, kchunk;
   bool wide;    // C and its rows are 16-byte aligned
   tile::Tiles tiles;
+  AheadPair ahead;  // weights of the products to come (unsplit products only)
 };
 
 template <int EPI>
@@ -92,6 +94,8 @@ template <int EPI, bool kSplit, typename S>
 __global__ void __launch_bounds__(S::kThreads, 2) k_pk_gemm(const PkGemm g) {
   extern __shared__ __attribute__((aligned(16))) char lds_raw[];
   auto& sh = *reinterpret_cast<tile::Lds<S>*>(lds_raw);
+  const int own = g.tiles.blocks();
+  if (!kSplit && (int)blockIdx.x >= own) return read_ahead(g.ahead, own);
   int tm, tn;
   if (!g.tiles.of(blockIdx.x, tm, tn)) return;
   const int n0 = tn * S::kTN, m0 = tm * S::kTM, z = blockIdx.y;
@@ -694,7 +698,8 @@ void launch_gemm(const PkGemm& g, int splits, hipStream_t s) {
     using S = decltype(shape);
     PkGemm h = g;
     h.tiles = tile::tiles_of<S>(g.M, g.N, (int64_t)g.M * g.kchunk * 2);
-    k_pk_gemm<EPI, kSplit, S><<<dim3(h.tiles.blocks(), splits), S::kThreads, sizeof(tile::Lds<S>), s>>>(h);
+    const int blocks = ahead_blocks(h.ahead, h.tiles.blocks(), S::kThreads);
+    k_pk_gemm<EPI, kSplit, S><<<dim3(blocks, splits), S::kThreads, sizeof(tile::Lds<S>), s>>>(h);
   });
 }
 
@@ -712,9 +717,9 @@ void launch_splitk(dim3 grid, const float* part, int splits, int m, int n, const
 // C = epi(A . Bt^T + bias), or (splits > 1) as `splits` K ranges through
 // `part` (splits x m x n floats) and k_pk_splitk.
 int gemm(const uint16_t* a, int lda, const uint16_t* bt, int ldb, const uint16_t* bias, uint16_t* c, int ldc, int m,
-         int n, int k, int epi, int splits, float* part, hipStream_t s) {
+         int n, int k, int epi, int splits, float* part, hipStream_t s, const AheadPair& ahead = {}) {
   const bool wide = aligned16(c) && ldc % 8 == 0;
-  const PkGemm g{a, bt, bias, c, part, 0.0f, lda, ldb, ldc, m, n, k / splits, wide, {}};
+  const PkGemm g{a, bt, bias, c, part, 0.0f, lda, ldb, ldc, m, n, k / splits, wide, {}, splits > 1 ? AheadPair{} : ahead};
   if (lda > kFarRows || ldb > kFarRows) {
     PkGemm f = g;
     f.kchunk = k;
@@ -745,9 +750,21 @@ int gemm(const uint16_t* a, int lda, const uint16_t* bt, int ldb, const uint16_t
 // One encoder product wider than d. Never split: at one window its smallest
 // tiles already fill half the chip, and the pass that sums the partials
 // would cost more than the other half gives.
+// The weights of the two products after it are read ahead behind it.
+struct EncWeights {
+  const uint16_t* w;
+  int n, k, splits;  // the product's n and k, and its K splits
+};
+EncWeights enc_ln_weights(const uint16_t* w, int rows, int k) { return {w, kD, k, pick_splits(rows, kD, k)}; }
 int enc_gemm(const uint16_t* a, int lda, const uint16_t* bt, const uint16_t* bias, uint16_t* c, int ldc, int m, int n,
-             int k, int epi, hipStream_t s) {
-  return gemm(a, lda, bt, k, bias, c, ldc, m, n, k, epi, 1, nullptr, s);
+             int k, int epi, hipStream_t s, const EncWeights& next, const EncWeights& then) {
+  AheadPair p{};
+  const EncWeights* e[2] = {&next, &then};
+  for (int i = 0; i < 2; ++i) {
+    const int group = e[i]->w ? tile::ahead_group(m, e[i]->n, e[i]->splits, (int64_t)m * (e[i]->k / e[i]->splits) * 2) : 0;
+    p.a[i] = Ahead{e[i]->w, group > 0 ? e[i]->n : 0, e[i]->k / 64, group > 0 ? group : 1};
+  }
+  return gemm(a, lda, bt, k, bias, c, ldc, m, n, k, epi, 1, nullptr, s, p);
 }
 
 struct ReduceLnArgs {
@@ -773,7 +790,7 @@ void launch_reduce_ln(const ReduceLnArgs& r, hipStream_t s) {
 int enc_gemm_ln(const uint16_t* a, int lda, const uint16_t* bt, int m, int k, float* part, uint16_t* x, float scale,
                 const uint16_t* ln1, const uint16_t* ln2, int normed_x, uint16_t* out_a, hipStream_t s) {
   const int splits = pick_splits(m, kD, k);
-  const PkGemm g{a, bt, nullptr, x, part, scale, lda, k, kD, m, kD, k / splits, true, {}};
+  const PkGemm g{a, bt, nullptr, x, part, scale, lda, k, kD, m, kD, k / splits, true, {}, {}};
   const uint16_t* b2 = ln2 ? ln2 + kD : nullptr;
   if (splits == 1) {
     launch_gemm<EPI_RESIDUAL, false>(g, 1, s);
@@ -910,19 +927,23 @@ int lfm25_pk_encoder(const lfm25_pk_layer* layers, int32_t n_layers, uint16_t* x
     const lfm25_pk_layer& L = layers[i];
     const uint16_t* next_ln = i + 1 < n_layers ? ln_of(layers[i + 1], 0) : nullptr;
     // Macaron FFN 1: x = bf16(x + FFN(a) / 2), a = LN_att(x)
-    PK_TRY(enc_gemm(a, kD, L.ff1_w1, nullptr, big, kPkFfn, rows, kPkFfn, kD, EPI_SWISH, s));
+    PK_TRY(enc_gemm(a, kD, L.ff1_w1, nullptr, big, kPkFfn, rows, kPkFfn, kD, EPI_SWISH, s,
+                    enc_ln_weights(L.ff1_w2, rows, kPkFfn), {L.qkv, 3 * kD, kD, 1}));
     PK_TRY(enc_gemm_ln(big, kPkFfn, L.ff1_w2, rows, kPkFfn, part, x, 0.5f, ln_of(L, 1), nullptr, 0, a, s));
     // relative-position self-attention: x = bf16(x + out(att)), a = LN_conv(x)
-    PK_TRY(enc_gemm(a, kD, L.qkv, L.qkv_bias, big, 3 * kD, rows, 3 * kD, kD, EPI_BIAS, s));
+    PK_TRY(enc_gemm(a, kD, L.qkv, L.qkv_bias, big, 3 * kD, rows, 3 * kD, kD, EPI_BIAS, s,
+                    enc_ln_weights(L.out, rows, kD), {L.pw1, 2 * kD, kD, 1}));
     k_pk_attention<<<dim3(kPkHeads, batch, kAttSplit), kAttBlockThreads, 0, s>>>(big, L.pos, L.att_delta, o, valid);
     PK_TRY(enc_gemm_ln(o, kD, L.out, rows, kD, part, x, 1.0f, ln_of(L, 2), nullptr, 0, a, s));
     // conv module: x = bf16(x + pw2(conv(pw1(a)))), a = LN_ff2(x)
-    PK_TRY(enc_gemm(a, kD, L.pw1, nullptr, big, 2 * kD, rows, 2 * kD, kD, EPI_NONE, s));
+    PK_TRY(enc_gemm(a, kD, L.pw1, nullptr, big, 2 * kD, rows, 2 * kD, kD, EPI_NONE, s,
+                    enc_ln_weights(L.pw2, rows, kD), {L.ff2_w1, kPkFfn, kD, 1}));
     k_pk_conv<<<dim3(kD / kConvCh, kAttT / kConvFrames, batch), kConvThreads, 0, s>>>(big, L.dw, L.dw_b, o, valid);
     PK_TRY(enc_gemm_ln(o, kD, L.pw2, rows, kD, part, x, 1.0f, ln_of(L, 3), nullptr, 0, a, s));
     // Macaron FFN 2 and the block's output norm: x = LN_out(bf16(x + FFN(a) / 2)),
     // a = LN_ff1 of the next layer (x)
-    PK_TRY(enc_gemm(a, kD, L.ff2_w1, nullptr, big, kPkFfn, rows, kPkFfn, kD, EPI_SWISH, s));
+    PK_TRY(enc_gemm(a, kD, L.ff2_w1, nullptr, big, kPkFfn, rows, kPkFfn, kD, EPI_SWISH, s,
+                    enc_ln_weights(L.ff2_w2, rows, kPkFfn), {i + 1 < n_layers ? layers[i + 1].ff1_w1 : nullptr, kPkFfn, kD, 1}));
     PK_TRY(enc_gemm_ln(big, kPkFfn, L.ff2_w2, rows, kPkFfn, part, x, 0.5f, ln_of(L, 4), next_ln, 1, a, s));
   }
 #undef PK_TRY

@@ -21,6 +21,7 @@
 // projection's output, norm, gate and residual, FP32 inside.
 #include <algorithm>
 
+#include "lfm25_ahead.h"
 #include "lfm25_gemm.h"
 #include "lfm25_host.h"
 #include "lfm25_layout.h"
@@ -120,6 +121,7 @@ struct PpGemm {
   uint16_t* c;        // [rows][ldc]
   int rows, n, k, ldc;
   tile::Tiles tiles;
+  AheadPair ahead;  // weights of the products to come
 };
 
 // PP_STORE: c = bf16(a . w^T). PP_RESIDUAL: c = bf16(c + bf16(a . w^T)) (the
@@ -131,6 +133,8 @@ template <int EPI, typename S>
 __global__ void __launch_bounds__(S::kThreads, 2) k_pp_gemm(const PpGemm g) {
   extern __shared__ __attribute__((aligned(16))) char lds_raw[];
   auto& sh = *reinterpret_cast<tile::Lds<S>*>(lds_raw);
+  const int own = g.tiles.blocks();
+  if ((int)blockIdx.x >= own) return read_ahead(g.ahead, own);
   int tm, tn;
   if (!g.tiles.of(blockIdx.x, tm, tn)) return;
   const int n0 = tn * S::kTN, m0 = tm * S::kTM;
@@ -178,7 +182,8 @@ void launch_gemm(PpGemm g, hipStream_t s) {
   tile::with_shape(g.rows, g.n, 1, [&](auto shape) {
     using S = decltype(shape);
     g.tiles = tile::tiles_of<S>(g.rows, g.n, (int64_t)g.rows * g.k * 2);
-    k_pp_gemm<EPI, S><<<g.tiles.blocks(), S::kThreads, sizeof(tile::Lds<S>), s>>>(g);
+    const int blocks = ahead_blocks(g.ahead, g.tiles.blocks(), S::kThreads);
+    k_pp_gemm<EPI, S><<<blocks, S::kThreads, sizeof(tile::Lds<S>), s>>>(g);
   });
 }
 
@@ -576,32 +581,40 @@ int prompt_layers(const lfm25_batch* b, const int32_t* tokens, const PromptRuns&
   p.capacity = b->capacity;
   p.vocab = b->vocab;
   const int norm_blocks = (rows + kNormRows - 1) / kNormRows;
+  // the n x k weights w of a product to come
+  const auto ahead = [&](const uint16_t* w, int n, int k, bool silu) {
+    const int group = tile::ahead_group(rows, n, 1, (int64_t)rows * k * 2) / (silu ? 2 : 1);
+    return Ahead{w, group > 0 ? n : 0, k / 64, group > 0 ? group : 1};
+  };
   k_pp_embed<<<norm_blocks, kNormRows * kWave, 0, s>>>(p, runs, tokens);
   for (int l = 0; l < kLayers; ++l) {
-    const bool attn = is_attn(l);
-    const uint16_t* w = p.weights + layer_off(l);
+    const bool attn = is_attn(l), next = is_attn(l + 1);
+    const uint16_t *w = p.weights + layer_off(l), *nw = p.weights + layer_off(l + 1);
     const auto tensor = [&](int a, int c) { return w + slot_off(attn, attn ? a : c); };
+    const uint16_t *w_out = tensor(A_O, C_OUT), *w_up = tensor(A_W1, C_W1), *w_down = tensor(A_W2, C_W2);
+    const Ahead out = ahead(w_out, kHidden, kHidden, false), up = ahead(w_up, 2 * kFfn, kHidden, true);
+    const Ahead down = ahead(w_down, kHidden, kFfn, false);
+    const Ahead mixer = l + 1 == kLayers ? Ahead{nullptr, 0, 1, 1}
+                        : ahead(nw + slot_off(next, next ? (int)A_Q : (int)C_IN), next ? 2 * kHidden : 3 * kHidden, kHidden, false);
     if (attn) {
       const int att = l - conv_before(l);
-      launch_gemm<PP_STORE>(PpGemm{p.xn, tensor(A_Q, 0), p.big, rows, 2 * kHidden, kHidden, 2 * kHidden, {}}, s);
+      launch_gemm<PP_STORE>(PpGemm{p.xn, tensor(A_Q, 0), p.big, rows, 2 * kHidden, kHidden, 2 * kHidden, {}, {{out, up}, 0}}, s);
       k_pp_qkv<<<rows, 256, 0, s>>>(p, l, att);
       // query positions per block: as many as still leave a block per CU
       if (rows >= 32 * 64) launch_attention<64>(p, runs, att, s);
       else if (rows >= 32 * 32) launch_attention<32>(p, runs, att, s);
       else launch_attention<16>(p, runs, att, s);
     } else {
-      launch_gemm<PP_STORE>(PpGemm{p.xn, tensor(0, C_IN), p.big, rows, 3 * kHidden, kHidden, 3 * kHidden, {}}, s);
+      launch_gemm<PP_STORE>(PpGemm{p.xn, tensor(0, C_IN), p.big, rows, 3 * kHidden, kHidden, 3 * kHidden, {}, {{out, up}, 0}}, s);
       k_pp_conv<<<(rows + 1) / 2, 256, 0, s>>>(p, l, conv_before(l));
     }
-    launch_gemm<PP_RESIDUAL>(PpGemm{p.y, tensor(A_O, C_OUT), p.x, rows, kHidden, kHidden, kHidden, {}}, s);
+    launch_gemm<PP_RESIDUAL>(PpGemm{p.y, w_out, p.x, rows, kHidden, kHidden, kHidden, {}, {}}, s);
     k_pp_norm<<<norm_blocks, kNormRows * kWave, 0, s>>>(p.x, tensor(A_FFNNORM, C_FFNNORM), p.xn, rows);
-    launch_gemm<PP_SILU>(PpGemm{p.xn, tensor(A_W1, C_W1), p.big, rows, 2 * kFfn, kHidden, kFfn, {}}, s);
-    launch_gemm<PP_RESIDUAL>(PpGemm{p.big, tensor(A_W2, C_W2), p.x, rows, kHidden, kFfn, kHidden, {}}, s);
-    if (l + 1 < kLayers) {
-      const bool next = is_attn(l + 1);
+    launch_gemm<PP_SILU>(PpGemm{p.xn, w_up, p.big, rows, 2 * kFfn, kHidden, kFfn, {}, {{down, mixer}, 0}}, s);
+    launch_gemm<PP_RESIDUAL>(PpGemm{p.big, w_down, p.x, rows, kHidden, kFfn, kHidden, {}, {}}, s);
+    if (l + 1 < kLayers)
       k_pp_norm<<<norm_blocks, kNormRows * kWave, 0, s>>>(
-          p.x, p.weights + layer_off(l + 1) + slot_off(next, next ? (int)A_OPNORM : (int)C_OPNORM), p.xn, rows);
-    }
+          p.x, nw + slot_off(next, next ? (int)A_OPNORM : (int)C_OPNORM), p.xn, rows);
   }
   *x = p.x;
   return check_launch("prompt pass");
