@@ -361,6 +361,9 @@ __global__ void __launch_bounds__(kWave) k_pk_reduce_ln(const float* __restrict_
 // q (scaled, bias_v folded in), k, v come from the q|k|v rows [T x 3072];
 // P_h^T is the head's [2T x 128] position table (last row zero).
 //
+// Two ways to split the work (launch_attention chooses).
+//
+// k_pk_attention: two blocks per (sequence, head).
 // The block first requests everything it reads (P, K and V into LDS, each
 // wave's 16 query rows into registers) in one round of 16-byte loads. Each
 // wave then forms its queries' position scores and key scores from LDS on
@@ -591,6 +594,187 @@ __global__ void __launch_bounds__(kAttBlockThreads, 1)
       *reinterpret_cast<u32x2_t*>(orow + 16 * dt) = pk;
     }
   }
+}
+
+// k_pk_attention_keys: a block takes 16 queries of one (sequence, head) and
+// its four waves split the keys, 32 each, so one window runs on 64 CUs
+// instead of 16. Bound by the latency of its one round of loads and of the
+// two meetings of the waves. Nothing but the values is used twice by a wave,
+// so keys, queries and the 48 rows of P_h^T that the shifted index
+// T-1-i+j spans for them go from memory straight into MFMA operands, all of a
+// block's loads in flight at once; the values are copied into the wave's LDS
+// and read back transposed. The waves meet for the rows' maxima, and to add
+// their partial values, which are divided by the rows' sums then.
+constexpr int kAkWaves = 4, kAkQueries = 16;
+constexpr int kAkThreads = kAkWaves * kWave;
+constexpr int kAkKeys = kAttT / kAkWaves;    // keys per wave
+constexpr int kAkBdRow = 48 + 4;             // bf16 per LDS row of a query's position scores
+constexpr int kAkOutRow = kDk + 4;           // floats per LDS row of a query's partial values
+struct PkAttKeysLds {
+  union {
+    uint4 v[kAkKeys * kDk / 8];              // the wave's values, then
+    float out[kAkQueries][kAkOutRow];        // its partial results
+  } w[kAkWaves];
+  uint16_t bd[kAkWaves][kAkQueries][kAkBdRow];
+  float top[kAkWaves][kAkQueries], sum[kAkWaves][kAkQueries];
+};
+
+// The transposing reads of 32 keys x 64 dimensions and the wait for them as
+// one statement (as in the prompt pass's attention, lfm25_prompt.hip).
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void read_values(const uint32_t (&a)[4], s16x4 (&lo)[4], s16x4 (&hi)[4]) {
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %8\n\t"
+      "ds_read_b64_tr_b16 %1, %9\n\t"
+      "ds_read_b64_tr_b16 %2, %10\n\t"
+      "ds_read_b64_tr_b16 %3, %11\n\t"
+      "ds_read_b64_tr_b16 %4, %8 offset:4096\n\t"
+      "ds_read_b64_tr_b16 %5, %9 offset:4096\n\t"
+      "ds_read_b64_tr_b16 %6, %10 offset:4096\n\t"
+      "ds_read_b64_tr_b16 %7, %11 offset:4096\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(lo[0]), "=&v"(lo[1]), "=&v"(lo[2]), "=&v"(lo[3]), "=&v"(hi[0]), "=&v"(hi[1]), "=&v"(hi[2]), "=&v"(hi[3])
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3])
+      : "memory");
+}
+
+__global__ void __launch_bounds__(kAkThreads, 2)
+    k_pk_attention_keys(const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ pos,
+                        const uint16_t* __restrict__ delta, uint16_t* __restrict__ out, int valid) {
+#if defined(__HIP_DEVICE_COMPILE__)  // (the host pass has no LDS address space)
+  __shared__ PkAttKeysLds sh;
+  constexpr int kDs = kDk / 32;  // steps of 32 dimensions
+  const int h = blockIdx.x, b = blockIdx.y, i0 = kAkQueries * blockIdx.z;
+  const int t = threadIdx.x, w = wave_id(), l = lane_id(), col = l & 15, g = l >> 4;
+  const uint16_t* base = qkv + (size_t)b * kAttT * 3 * kD + h * kDk;
+  // values: key row r's chunk c in slot 16 r + (c ^ 2 (r % 8))
+  {
+    const uint16_t* v = base + 2 * kD + (size_t)kAkKeys * w * 3 * kD;
+#pragma unroll
+    for (int i = 0; i < kAkKeys * kDk / 8 / kWave; ++i) {
+      const int slot = i * kWave + l, r = slot / 16, c = (slot % 16) ^ (2 * (r & 7));
+      __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)(v + (size_t)r * 3 * kD + 8 * c),
+                                       (tile::LdsVoid*)&sh.w[w].v[i * kWave], 16, 0, 0);
+    }
+  }
+  uint4 q[kDs], k[2][kDs], p[3][kDs];
+  const int p0 = kAttT - kAkQueries - i0 + kAkKeys * w;  // T-1-i+j of the last query and the wave's first key
+#pragma unroll
+  for (int ds = 0; ds < kDs; ++ds) {
+    const int d = 32 * ds + 8 * g;
+    q[ds] = *reinterpret_cast<const uint4*>(base + (size_t)(i0 + col) * 3 * kD + d);
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+      k[kt][ds] = *reinterpret_cast<const uint4*>(base + kD + (size_t)(kAkKeys * w + 16 * kt + col) * 3 * kD + d);
+#pragma unroll
+    for (int pt = 0; pt < 3; ++pt)
+      p[pt][ds] = *reinterpret_cast<const uint4*>(pos + ((size_t)h * 2 * kAttT + p0 + 16 * pt + col) * kDk + d);
+  }
+  // position scores of query i0 + col and rows 16 pt + 4 g + e of the slice
+#pragma unroll
+  for (int pt = 0; pt < 3; ++pt) {
+    f32x4_t a{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int ds = 0; ds < kDs; ++ds)
+      a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(p[pt][ds]), as_bf16x8(q[ds]), a, 0, 0, 0);
+    *reinterpret_cast<uint2*>(&sh.bd[w][col][16 * pt + 4 * g]) =
+        uint2{tile::pack_pair(a[0], a[1]), tile::pack_pair(a[2], a[3])};
+  }
+  // key scores: s[kt][e] of key 32 w + 16 kt + 4 g + e and query i0 + col
+  f32x4_t s[2] = {f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+  for (int ds = 0; ds < kDs; ++ds) {
+    const uint4 dl = *reinterpret_cast<const uint4*>(delta + h * kDk + 32 * ds + 8 * g);
+    const uint32_t dw[4] = {dl.x, dl.y, dl.z, dl.w}, qw[4] = {q[ds].x, q[ds].y, q[ds].z, q[ds].w};
+    uint32_t u[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) u[e] = tile::pack_pair(lo_f32(qw[e]) + lo_f32(dw[e]), hi_f32(qw[e]) + hi_f32(dw[e]));
+    const bf16x8_t qu = as_bf16x8(uint4{u[0], u[1], u[2], u[3]});
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+      s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(k[kt][ds]), qu, s[kt], 0, 0, 0);
+  }
+  // position term and mask, then the rows' maxima over the waves
+  float top = -INFINITY;
+#pragma unroll
+  for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int j = 16 * kt + 4 * g + e;
+      float v = s[kt][e] + bf16_to_f32(sh.bd[w][col][15 - col + j]);
+      if (kAkKeys * w + j >= valid) v = -INFINITY;
+      s[kt][e] = v;
+      top = fmaxf(top, v);
+    }
+  top = max_lanes16(top);
+  if (l < 16) sh.top[w][l] = top;
+  lds_barrier();
+#pragma unroll
+  for (int u = 0; u < kAkWaves; ++u) top = fmaxf(top, sh.top[u][col]);
+  float z = 0.0f;
+  uint32_t hw[4], lw[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float e0 = expf(s[i / 2][2 * (i % 2)] - top), e1 = expf(s[i / 2][2 * (i % 2) + 1] - top);
+    z += e0 + e1;
+    hw[i] = tile::pack_pair(e0, e1);
+    lw[i] = tile::pack_pair(e0 - lo_f32(hw[i]), e1 - hi_f32(hw[i]));
+  }
+  z = sum_lanes16(z);
+  if (l < 16) sh.sum[w][l] = z;
+  const bf16x8_t hi = as_bf16x8(uint4{hw[0], hw[1], hw[2], hw[3]}), lo = as_bf16x8(uint4{lw[0], lw[1], lw[2], lw[3]});
+  // o^T = V^T . e^T over the wave's keys: a lane's eight k values are the keys
+  // {4 g + e, 16 + 4 g + e} in both operands
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the wave's own value copies
+  f32x4_t o[kDk / 16];
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {
+    uint32_t at[4];
+    const int vr = 4 * g + col / 4;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+      at[dt] = (uint32_t)(uintptr_t)(tile::LdsVoid*)&sh.w[w].v[16 * vr + ((8 * half + 2 * dt + (l & 3) / 2) ^ (2 * (vr & 7)))] + 8 * (l & 1);
+    s16x4 v0[4], v1[4];
+    read_values(at, v0, v1);
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) {
+      const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(v0[dt], v1[dt], 0, 1, 2, 3, 4, 5, 6, 7));
+      f32x4_t a{0.0f, 0.0f, 0.0f, 0.0f};
+      a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, hi, a, 0, 0, 0);
+      o[4 * half + dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, lo, a, 0, 0, 0);
+    }
+  }
+  // (over the wave's own values, which it has read)
+#pragma unroll
+  for (int dt = 0; dt < kDk / 16; ++dt) *reinterpret_cast<f32x4_t*>(&sh.w[w].out[col][16 * dt + 4 * g]) = o[dt];
+  lds_barrier();
+  // the waves' partials in order, over the row's sum: eight dimensions per thread
+  const int qi = t / 16, d0 = 8 * (t % 16);
+  float total = sh.sum[0][qi], v[8];
+#pragma unroll
+  for (int u = 1; u < kAkWaves; ++u) total += sh.sum[u][qi];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    v[e] = sh.w[0].out[qi][d0 + e];
+#pragma unroll
+    for (int u = 1; u < kAkWaves; ++u) v[e] += sh.w[u].out[qi][d0 + e];
+    v[e] /= total;
+  }
+  tile::store_bf16<8>(out + (size_t)(b * kAttT + i0 + qi) * kD + h * kDk + d0, v, false);
+#endif
+}
+
+// Blocks of 16 queries while they fit the chip twice (two of them to a CU):
+// 6.4 us against 10.5 at one window, 6.7 / 10.7 at four, 9.9 / 11.4 at eight;
+// at ten windows their third round makes it 12.7 against 11.1, at sixteen
+// 16.0 against 11.8.
+void launch_attention(const uint16_t* qkv, const uint16_t* pos, const uint16_t* delta, uint16_t* out, int batch,
+                      int valid, hipStream_t s) {
+  constexpr int kKeysBlocks = kPkHeads * (kAttT / kAkQueries);
+  if (batch <= 2 * tile::kCus / kKeysBlocks)
+    k_pk_attention_keys<<<dim3(kPkHeads, batch, kAttT / kAkQueries), kAkThreads, 0, s>>>(qkv, pos, delta, out, valid);
+  else
+    k_pk_attention<<<dim3(kPkHeads, batch, kAttSplit), kAttBlockThreads, 0, s>>>(qkv, pos, delta, out, valid);
 }
 
 // ------------------------------------------------------------------ conv module
@@ -866,8 +1050,7 @@ int lfm25_pk_attention(const uint16_t* qkv, const uint16_t* pos, const uint16_t*
   LFM25_REQUIRE(batch >= 1 && valid >= 1 && valid <= frames, "pk attention: need batch >= 1 and 1 <= valid <= frames");
   LFM25_REQUIRE(aligned16(qkv) && aligned16(pos) && aligned16(delta) && (reinterpret_cast<uintptr_t>(out) & 7) == 0,
                 "pk attention: qkv, pos, delta must be 16-byte and out 8-byte aligned");
-  k_pk_attention<<<dim3(kPkHeads, batch, kAttSplit), kAttBlockThreads, 0, reinterpret_cast<hipStream_t>(stream)>>>(qkv, pos, delta,
-                                                                                                  out, valid);
+  launch_attention(qkv, pos, delta, out, batch, valid, reinterpret_cast<hipStream_t>(stream));
   return check_launch("parakeet attention");
 }
 
@@ -933,7 +1116,7 @@ int lfm25_pk_encoder(const lfm25_pk_layer* layers, int32_t n_layers, uint16_t* x
     // relative-position self-attention: x = bf16(x + out(att)), a = LN_conv(x)
     PK_TRY(enc_gemm(a, kD, L.qkv, L.qkv_bias, big, 3 * kD, rows, 3 * kD, kD, EPI_BIAS, s,
                     enc_ln_weights(L.out, rows, kD), {L.pw1, 2 * kD, kD, 1}));
-    k_pk_attention<<<dim3(kPkHeads, batch, kAttSplit), kAttBlockThreads, 0, s>>>(big, L.pos, L.att_delta, o, valid);
+    launch_attention(big, L.pos, L.att_delta, o, batch, valid, s);
     PK_TRY(enc_gemm_ln(o, kD, L.out, rows, kD, part, x, 1.0f, ln_of(L, 2), nullptr, 0, a, s));
     // conv module: x = bf16(x + pw2(conv(pw1(a)))), a = LN_ff2(x)
     PK_TRY(enc_gemm(a, kD, L.pw1, nullptr, big, 2 * kD, rows, 2 * kD, kD, EPI_NONE, s,
