@@ -175,5 +175,13 @@ def check(rc: int, what: str) -> None:
     raise RuntimeError(f"{what}: {msg}")
 
 
+_functions = {}  # name -> the library's function, from its first call on
+
+
 def call(name: str, *args) -> None:
-    check(getattr(load(), name)(*args), name)
+    fn = _functions.get(name)
+    if fn is None:
+        fn = _functions[name] = getattr(load(), name)
+    rc = fn(*args)
+    if rc != LFM25_OK:
+        check(rc, name)

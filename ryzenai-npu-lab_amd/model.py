@@ -29,7 +29,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .batch import PROMPT_ROWS, PromptWorkspace, run_pass, run_prompt
+from .batch import PROMPT_ROWS, PromptWorkspace, check_tokens, device_tokens, run_pass, run_prompt
 from .bf16 import bf16_bits_to_f32
 from .weights import (HEAD_DIM, HIDDEN, KINDS, KV_HEADS, VOCAB, load_safetensors, pack_stream, pack_w8,
                       rope_table, synthetic_checkpoint)
@@ -144,13 +144,11 @@ class X8Model:
         _lib.call("lfm25_decoder_reset", self._desc, self._stream())
 
     def _run(self, tokens, n_gen: int) -> list[int]:
-        tokens = [int(t) for t in tokens]
+        tokens = list(map(int, tokens))
         steps = len(tokens) + max(n_gen - 1, 0)
         if self.position + steps > self.capacity:
             raise ValueError(f"KV capacity {self.capacity} reached")
-        for t in tokens:
-            if not 0 <= t < self.vocab:
-                raise ValueError(f"token id {t} outside the vocabulary")
+        check_tokens(tokens, self.vocab)
         if len(tokens) > self._tokens_in.numel() or n_gen > self._tokens_out.numel():
             raise ValueError("too many tokens for one call")
         src = torch.tensor(tokens, dtype=torch.int32)
@@ -192,9 +190,7 @@ class X8Model:
     def _check_tokens(self, tokens, steps: int) -> None:
         if self.position + steps > self.capacity:
             raise ValueError(f"KV capacity {self.capacity} reached")
-        for t in tokens:
-            if not 0 <= int(t) < self.vocab:
-                raise ValueError(f"token id {t} outside the vocabulary")
+        check_tokens(tokens, self.vocab)
 
     def _prompt(self, token_ids, n_gen: int) -> list[int]:
         """A prompt and n_gen greedy tokens, the way the reference's prefill
@@ -203,7 +199,7 @@ class X8Model:
         PROMPT_ROWS tokens lfm25_batch_pass; at most PB tokens go token by
         token, one launch beating a pass), then the other tokens in one
         decode call, which reads the first on the device."""
-        tokens = [int(t) for t in token_ids]
+        tokens = list(map(int, token_ids))
         self._check_tokens(tokens, len(tokens) + max(n_gen - 1, 0))
         rows = len(tokens)
         if rows <= PB or not self.batched_prefill:
@@ -216,11 +212,11 @@ class X8Model:
             first = self._selected[rows - 1:rows]
         else:
             hidden = torch.empty(HIDDEN, dtype=torch.bfloat16, device=self.device)
-            ids = torch.tensor(tokens, dtype=torch.int32).to(self.device)
+            ids = device_tokens(tokens, self.device)
             run_prompt(batch, self._prompt_ws, ids, [(0, self.position, rows)], self._selected, self._stream(), hidden)
             first = self._selected[:1]
         self.position += rows
-        self.ctl[_lib.CTL_POSITION] = self.position
+        self.ctl[_lib.CTL_POSITION].fill_(self.position)  # (an assignment waits for the stream)
         self.ctl[_lib.CTL_TOKEN:_lib.CTL_TOKEN + 1].copy_(first)  # what a decode without tokens_in continues from
         if n_gen > 1:
             _lib.call("lfm25_decode", self._desc, first.data_ptr(), 1, n_gen - 1, self._tokens_out.data_ptr(),
