@@ -13,9 +13,10 @@
 //   +append, attention -> out_proj+residual -> norm + w1/w3+SiLU gate ->
 //   w2+residual -> (select) final norm + head GEMM + per-block argmax -> pick
 //
-// GEMM kernels: a block owns NT tiles of 16 weight rows and all batch rows;
+// GEMM kernels: a block owns NT tiles of 16 weight rows and MT tiles of 16
+// batch rows (launch_pass chooses MT; blockIdx.y is the group of 16 MT rows);
 // its 8 waves split (tile, K slice), each wave streams its 16 x (K / KS)
-// weight slice with 16-byte buffer loads and multiplies it into four 16 x 16
+// weight slice with 16-byte buffer loads and multiplies it into MT 16 x 16
 // f32 accumulators (one per 16 batch rows) with v_mfma_f32_16x16x32_bf16; the
 // KS partial sums of a tile meet in LDS, summed in slice order, and the
 // epilogue of the phase (conv gate, residual, SiLU gate, QK-norm + RoPE + KV
@@ -60,7 +61,7 @@ constexpr size_t kBwCtl = 0;                                     // int32 [64]: 
 constexpr size_t kBwRows = 256;                                  // int32 [64][4] row table
 constexpr size_t kBwStart = kBwRows + kRowsMax * 16;             // int32 [64] decode start positions
 constexpr size_t kBwX = 2048;                                    // bf16 [64][1024] residual stream
-constexpr size_t kBwXn = kBwX + (size_t)kRowsMax * kHidden * 2;  // bf16 [64][1024] normed rows (above kFoldRows)
+constexpr size_t kBwXn = kBwX + (size_t)kRowsMax * kHidden * 2;  // bf16 [64][1024] normed rows (k_bx_norm)
 constexpr size_t kBwG = kBwXn + (size_t)kRowsMax * kHidden * 2;  // bf16 [64][2560] FFN gate values
 constexpr size_t kBwY = kBwG + (size_t)kRowsMax * kFfn * 2;      // bf16 [64][1024] conv out / context
 constexpr size_t kBwQ = kBwY + (size_t)kRowsMax * kHidden * 2;   // bf16 [64][1024] queries
@@ -68,8 +69,8 @@ constexpr size_t kBwCand = kBwQ + (size_t)kRowsMax * kHidden * 2;  // u64 [head 
 constexpr int kHeadBlocksMax = 256;  // head blocks (kHeadBlocks)
 constexpr int kResSplit = 4;  // K slices of a split residual projection (one block each)
 constexpr size_t kBwPart = kBwCand + (size_t)kHeadBlocksMax * kRowsMax * 8;  // f32 [64 tiles][4][64 rows][16]
-constexpr size_t kBwCount = kBwPart + (size_t)(kHidden / 16) * kResSplit * kRowsMax * 16 * 4;  // int32 [64 tiles]
-constexpr size_t kBwBytes = kBwCount + (size_t)(kHidden / 16) * 4;
+constexpr size_t kBwCount = kBwPart + (size_t)(kHidden / 16) * kResSplit * kRowsMax * 16 * 4;  // int32 [64 tiles][4]
+constexpr size_t kBwBytes = kBwCount + (size_t)(kHidden / 16) * kMT * 4;
 // The persistent batched decode's exchange region follows, on a 256-byte
 // boundary (batch_persistent_bytes(), lfm25_decode.hip).
 constexpr size_t kBwPersist = (kBwBytes + 255) & ~(size_t)255;
@@ -133,20 +134,22 @@ __device__ __forceinline__ bf16x8_t load_bf16x8(Rsrc r, int voff, int soff) {
 // Partial tiles of the 8 waves: part[w][m][lane][e] holds, for wave w's tile
 // and 16-row batch tile m, the f32 accumulator element e of `lane` (row
 // 4 (lane / 16) + e of the weight tile, batch row 16 m + lane % 16).
+template <int MT>
 struct GemmLds {
-  f32x4_t part[kGW][kMT][kWave];
+  f32x4_t part[kGW][MT][kWave];
 };
 // The same after a staged product (gemm_tiles_staged): the batch's rows in
 // LDS first (padded to kXRow bytes, so that the lanes' 16-byte reads hit
 // distinct banks), the partial tiles in the same space once every product
 // has read them.
 constexpr int kXRow = kHidden * 2 + 16;
+template <int MT>
 struct GemmLdsStaged {
   union {
-    char x[kRowsMax][kXRow];
-    f32x4_t part[kGW][kMT][kWave];
+    char x[16 * MT][kXRow];
+    f32x4_t part[kGW][MT][kWave];
   };
-  float ss[kRowsMax][2];  // the rows' sums of squares, per half (RowStage)
+  float ss[16 * MT][2];  // the rows' sums of squares, per half (RowStage)
 };
 
 // The batch tiles in use (rows past `rows` as zeros) staged into LDS rows of
@@ -155,23 +158,24 @@ struct GemmLdsStaged {
 // copies the 8 elements of column block t % 128 of rows t / 128 + 4j of every
 // tile, so waves 2q and 2q + 1 cover one row: the row's mean square is the
 // sum of their two wave sums (each vector's 8 squares added in element
-// order, then the wave's tree), in that order. Above that every block would
-// repeat too much of the norm (it sits between the loads and the products),
-// so k_bx_norm writes the normed rows once and they are copied as they are.
+// order, then the wave's tree), in that order. Above that (the head), or
+// where the caller says so, they were normed by k_bx_norm and are copied as
+// they are.
 // load() requests the rows and the thread's 8 norm weights; store() (every
 // thread of the block) waits for them, exchanges the half-row sums through
 // LDS (one block barrier) and writes the rows; the caller's barrier then
 // publishes them.
 constexpr int kFoldRows = 16;
+template <int MT>
 struct RowStage {
   static constexpr int kPerTile = 16 * (kHidden / 8) / kGT;  // 4 vectors per thread per batch tile
-  u32x4_t v[kMT][kPerTile];
+  u32x4_t v[MT][kPerTile];
   u32x4_t g;
-  __device__ __forceinline__ void load(const uint16_t* x, const uint16_t* gamma, int rows, int mt) {
+  __device__ __forceinline__ void load(const uint16_t* x, const uint16_t* gamma, int rows, int mt, bool fold) {
     const Rsrc rx = rsrc(x, (size_t)rows * kHidden * 2);
-    if (rows <= kFoldRows) g = reinterpret_cast<const u32x4_t*>(gamma)[threadIdx.x % (kHidden / 8)];
+    if (fold) g = reinterpret_cast<const u32x4_t*>(gamma)[threadIdx.x % (kHidden / 8)];
 #pragma unroll
-    for (int k = 0; k < kMT; ++k) {
+    for (int k = 0; k < MT; ++k) {
       if (k < mt) {
 #pragma unroll
         for (int j = 0; j < kPerTile; ++j)
@@ -184,7 +188,7 @@ struct RowStage {
   __device__ __forceinline__ void store(char (*xl)[kXRow], float (*ssl)[2], int mt, bool fold) {
     if (!fold) {
 #pragma unroll
-      for (int k = 0; k < kMT; ++k) {
+      for (int k = 0; k < MT; ++k) {
         if (k < mt) {
 #pragma unroll
           for (int j = 0; j < kPerTile; ++j) *reinterpret_cast<u32x4_t*>(&xl[row(k, j)][2 * col()]) = v[k][j];
@@ -194,7 +198,7 @@ struct RowStage {
     }
     const int half = wave_id() & 1;
 #pragma unroll
-    for (int k = 0; k < kMT; ++k) {
+    for (int k = 0; k < MT; ++k) {
       if (k < mt) {
 #pragma unroll
         for (int j = 0; j < kPerTile; ++j) {
@@ -211,7 +215,7 @@ struct RowStage {
     }
     lds_barrier();
 #pragma unroll
-    for (int k = 0; k < kMT; ++k) {
+    for (int k = 0; k < MT; ++k) {
       if (k < mt) {
 #pragma unroll
         for (int j = 0; j < kPerTile; ++j) {
@@ -246,8 +250,8 @@ struct NoMid {
   __device__ void operator()() const {}
 };
 // (KLen < K: the product over columns [k0, k0 + KLen) of rows of length K.)
-template <int NT, int KS, int K, typename Mid = NoMid, int KLen = K>
-__device__ __forceinline__ void gemm_tiles(const uint16_t* const* wt, const uint16_t* x, int rows, GemmLds& sh,
+template <int NT, int KS, int K, int MT, typename Mid = NoMid, int KLen = K>
+__device__ __forceinline__ void gemm_tiles(const uint16_t* const* wt, const uint16_t* x, int rows, GemmLds<MT>& sh,
                                            const Mid& mid = Mid{}, int k0 = 0) {
   static_assert(NT * KS <= kGW && KLen % (32 * KS) == 0 && K % KLen == 0, "tile split");
   constexpr int kSteps = KLen / (32 * KS);
@@ -262,9 +266,9 @@ __device__ __forceinline__ void gemm_tiles(const uint16_t* const* wt, const uint
   const Rsrc ra = rsrc(wt[t], (size_t)16 * K * 2);
   const Rsrc rb = rsrc(x, (size_t)rows * K * 2);
   const int a_off = ((l & 15) * K + 8 * (l >> 4)) * 2;
-  f32x4_t acc[kMT];
+  f32x4_t acc[MT];
 #pragma unroll
-  for (int m = 0; m < kMT; ++m) acc[m] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int m = 0; m < MT; ++m) acc[m] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
   bf16x8_t a[kSteps];
 #pragma unroll
   for (int st = 0; st < kSteps; ++st) a[st] = load_bf16x8(ra, a_off, (col0 + 32 * st) * 2);
@@ -283,7 +287,7 @@ __device__ __forceinline__ void gemm_tiles(const uint16_t* const* wt, const uint
   __builtin_amdgcn_sched_barrier(0);
   mid();
 #pragma unroll
-  for (int m = 0; m < kMT; ++m) {
+  for (int m = 0; m < MT; ++m) {
     if (m < mt) {
       if (m + 1 < mt) load_b(m + 1, bv[(m + 1) & 1]);
 #pragma unroll
@@ -292,7 +296,7 @@ __device__ __forceinline__ void gemm_tiles(const uint16_t* const* wt, const uint
     }
   }
 #pragma unroll
-  for (int m = 0; m < kMT; ++m) sh.part[w][m][l] = acc[m];
+  for (int m = 0; m < MT; ++m) sh.part[w][m][l] = acc[m];
 }
 
 // Reduced element (tile t, weight row i, batch row m) after gemm_tiles and a
@@ -306,8 +310,8 @@ __device__ __forceinline__ float gemm_at(const Lds& sh, int t, int i, int m) {
   return v;
 }
 
-// gemm_tiles for K = 1,024 over the RMSNorm of the residual stream x with
-// norm weights gamma, the normed activations staged in LDS (RowStage): every
+// gemm_tiles for K = 1,024 and the batch rows from m0 over the RMSNorm of the
+// residual stream x with norm weights gamma (formed here if kFold), the normed activations staged in LDS (RowStage): every
 // wave reads its B operands from there, so a K slice shared by NT tiles
 // crosses the vector cache once instead of NT times (at 64 rows the
 // activation reads, not the weights, bound the per-CU load rate), and no
@@ -319,11 +323,10 @@ struct DenseRows {
   __device__ static int off(int, int i) { return i; }
   __device__ static int span(int) { return 16; }
 };
-template <int NT, int KS, typename RowMap = DenseRows, typename Mid = NoMid>
+template <int NT, int KS, int MT, bool kFold, typename RowMap = DenseRows, typename Mid = NoMid>
 __device__ __forceinline__ void gemm_tiles_staged(const uint16_t* const* wt, const BatchParams& p, const uint16_t* gamma,
-                                                  GemmLdsStaged& sh, const Mid& mid = Mid{}) {
-  const int rows = p.rows;
-  const bool fold = rows <= kFoldRows;
+                                                  GemmLdsStaged<MT>& sh, int m0, const Mid& mid = Mid{}) {
+  const int rows = min(p.rows - m0, 16 * MT);
   constexpr int K = kHidden;
   static_assert(NT * KS <= kGW && K % (32 * KS) == 0, "tile split");
   constexpr int kSteps = K / (32 * KS);
@@ -332,8 +335,8 @@ __device__ __forceinline__ void gemm_tiles_staged(const uint16_t* const* wt, con
   const int t = w / KS, s = w % KS;
   const int mt = (rows + 15) / 16;
   const int col0 = s * (K / KS);
-  RowStage stage;
-  stage.load(fold ? b_x(p) : b_xn(p), gamma, rows, mt);
+  RowStage<MT> stage;
+  stage.load((kFold ? b_x(p) : b_xn(p)) + (size_t)m0 * kHidden, gamma, rows, mt, kFold);
   bf16x8_t a[kSteps];
   {
     const Rsrc ra = rsrc(wt[active ? t : 0], active ? (size_t)RowMap::span(t) * K * 2 : 0);
@@ -343,14 +346,14 @@ __device__ __forceinline__ void gemm_tiles_staged(const uint16_t* const* wt, con
   }
   __builtin_amdgcn_sched_barrier(0);
   mid();
-  stage.store(sh.x, sh.ss, mt, fold);
+  stage.store(sh.x, sh.ss, mt, kFold);
   lds_barrier();
-  f32x4_t acc[kMT];
+  f32x4_t acc[MT];
 #pragma unroll
-  for (int m = 0; m < kMT; ++m) acc[m] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int m = 0; m < MT; ++m) acc[m] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
   if (active) {
 #pragma unroll
-    for (int m = 0; m < kMT; ++m) {
+    for (int m = 0; m < MT; ++m) {
       if (m < mt) {
         const char* xr = &sh.x[16 * m + (l & 15)][2 * col0 + 16 * (l >> 4)];
 #pragma unroll
@@ -363,7 +366,7 @@ __device__ __forceinline__ void gemm_tiles_staged(const uint16_t* const* wt, con
   lds_barrier();  // every product has read the rows before the partial tiles overwrite them
   if (active) {
 #pragma unroll
-    for (int m = 0; m < kMT; ++m) sh.part[w][m][l] = acc[m];
+    for (int m = 0; m < MT; ++m) sh.part[w][m][l] = acc[m];
   }
 }
 
@@ -395,7 +398,7 @@ __global__ void __launch_bounds__(kWave) k_bx_embed(BatchParams p, const int32_t
 }
 
 // RMSNorm of every row (Lfm2RMSNorm.forward, modeling_lfm2.py:54-59, two
-// roundings), for passes of more than kFoldRows rows: 128 threads per row,
+// roundings), for the products that do not form it themselves: 128 threads per row,
 // thread j holding the 8 elements of column block j, with RowStage's order of
 // additions (each block's squares in element order, the wave sums of blocks
 // 0..63 and 64..127, then their sum), so a row's normed values are the same
@@ -439,21 +442,22 @@ struct Conv8Rows {
   __device__ static int off(int t, int i) { return t == 0 && i >= 8 ? kHidden + i - 8 : i; }
   __device__ static int span(int t) { return t == 0 ? kHidden + 8 : 8; }
 };
+template <int MT, bool kFold>
 __global__ void __launch_bounds__(kGT) k_bx_conv(BatchParams p, int l) {
-  __shared__ GemmLdsStaged sh;
+  __shared__ GemmLdsStaged<MT> sh;
   constexpr int kCh = 8;
-  __shared__ float bxs[kCh][kRowsMax];
-  __shared__ float cgs[kCh][kRowsMax];
-  __shared__ float win[kCh][kRowsMax][2];
-  static_assert(kRowsMax * kCh == kGT, "one (channel, row) per thread");
-  const int c0 = kCh * blockIdx.x;
-  const int n = kCh * p.rows;
+  __shared__ float bxs[kCh][16 * MT];
+  __shared__ float cgs[kCh][16 * MT];
+  __shared__ float win[kCh][16 * MT][2];
+  static_assert(16 * MT * kCh <= kGT, "one (channel, row) per thread");
+  const int c0 = kCh * blockIdx.x, m0 = 16 * MT * blockIdx.y;
+  const int n = kCh * min(p.rows - m0, 16 * MT);
   const int ci = conv_before(l);
   // The epilogue's operands: the thread's row and taps before the weights,
   // the conv state (addressed by the row) once the weights are requested.
   const int e = min((int)threadIdx.x, n - 1);
   const int i = e % kCh, m = e / kCh;
-  const RowInfo ri = b_row(p, m);
+  const RowInfo ri = b_row(p, m0 + m);
   uint16_t tap[kConvTaps], s1, s2;
   {
     const uint16_t* cw = conv_tensor<C_CONVW>(p.weights, l) + (c0 + i) * kConvTaps;
@@ -467,7 +471,7 @@ __global__ void __launch_bounds__(kGT) k_bx_conv(BatchParams p, int l) {
   };
   const uint16_t* w_in = conv_tensor<C_IN>(p.weights, l);
   const uint16_t* wt[2] = {w_in + (size_t)c0 * kHidden, w_in + (size_t)(2 * kHidden + c0) * kHidden};
-  gemm_tiles_staged<2, 4, Conv8Rows>(wt, p, conv_tensor<C_OPNORM>(p.weights, l), sh, states);
+  gemm_tiles_staged<2, 4, MT, kFold, Conv8Rows>(wt, p, conv_tensor<C_OPNORM>(p.weights, l), sh, m0, states);
   __syncthreads();
   const bool live = (int)threadIdx.x < n;
   if (live) {
@@ -487,7 +491,7 @@ __global__ void __launch_bounds__(kGT) k_bx_conv(BatchParams p, int l) {
     const float p1 = round_bf16(b * bf16_to_f32(tap[1]));
     const float p2 = round_bf16(bx * bf16_to_f32(tap[2]));
     const float c = round_bf16((p0 + p1) + p2);
-    b_y(p)[(size_t)m * kHidden + c0 + i] = f32_to_bf16(round_bf16(cgs[i][m] * c));
+    b_y(p)[(size_t)(m0 + m) * kHidden + c0 + i] = f32_to_bf16(round_bf16(cgs[i][m] * c));
     win[i][m][0] = a;
     win[i][m][1] = b;
   }
@@ -503,7 +507,7 @@ __global__ void __launch_bounds__(kGT) k_bx_conv(BatchParams p, int l) {
 // Residual projection of 16 output rows n0 .. n0 + 15: X[m][n] =
 // bf16(X[m][n] + bf16(W[n] . in[m])) (out_proj / o_proj with K = 1024, w2 with
 // K = 2560; the residual add of Lfm2DecoderLayer.forward, modeling_lfm2.py:431).
-// S blocks per tile (block b: tile b % 64, K slice b / 64), so that S times
+// S blocks per tile and row group (block b: tile b % 64, K slice b / 64), so that S times
 // as many CUs share the weights and, above all, the activations (at 64 rows
 // a tile reads 128-320 KB of them, which one CU's vector cache takes ~10 us
 // to pass); each publishes its partial tile at device scope and counts
@@ -519,17 +523,17 @@ __global__ void __launch_bounds__(kGT) k_bx_conv(BatchParams p, int l) {
 // memory model without its L2 writeback and invalidate, which only matter
 // for data written or read through an XCD's L2.
 constexpr int res_ks(int len) { return len % (32 * kGW) == 0 ? kGW : len % (32 * 5) == 0 ? 5 : 4; }
-template <int K, int S>
+template <int K, int S, int MT>
 __global__ void __launch_bounds__(kGT) k_bx_residual(BatchParams p, const uint16_t* w, const uint16_t* in) {
-  __shared__ GemmLds sh;
+  __shared__ GemmLds<MT> sh;
   __shared__ int last;
-  constexpr int kPer = kRowsMax * 16 / kGT;  // elements per thread
+  constexpr int kPer = (16 * MT * 16 + kGT - 1) / kGT;  // elements per thread
   constexpr int kLen = K / S, KS = res_ks(kLen);
   constexpr int kTiles = kHidden / 16;
   const int tile = blockIdx.x % kTiles, sp = blockIdx.x / kTiles;
-  const int n0 = 16 * tile;
-  const int n = 16 * p.rows;
-  uint16_t* x = b_x(p);
+  const int n0 = 16 * tile, m0 = 16 * MT * blockIdx.y;
+  const int rows = min(p.rows - m0, 16 * MT), n = 16 * rows;
+  uint16_t* x = b_x(p) + (size_t)m0 * kHidden;
   // the residual values, requested before the weights
   uint16_t h[kPer];
 #pragma unroll
@@ -538,10 +542,11 @@ __global__ void __launch_bounds__(kGT) k_bx_residual(BatchParams p, const uint16
     h[k] = x[(size_t)(e >> 4) * kHidden + n0 + (e & 15)];
   }
   const uint16_t* wt[1] = {w + (size_t)n0 * K};
-  gemm_tiles<1, KS, K, NoMid, kLen>(wt, in, p.rows, sh, NoMid{}, sp * kLen);
+  gemm_tiles<1, KS, K, MT, NoMid, kLen>(wt, in + (size_t)m0 * K, rows, sh, NoMid{}, sp * kLen);
   __syncthreads();
   // partial tile [m][i] of slice sp, then the count
-  float* part = b_part(p) + (size_t)tile * S * kRowsMax * 16;
+  float* part = b_part(p) + ((size_t)tile * S * kRowsMax + m0) * 16;
+  int32_t* count = b_count(p) + kMT * tile + blockIdx.y;
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
     const int e = threadIdx.x + kGT * k;
@@ -550,10 +555,10 @@ __global__ void __launch_bounds__(kGT) k_bx_residual(BatchParams p, const uint16
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this thread's partials have reached device scope
   __syncthreads();
   if (threadIdx.x == 0)
-    last = __hip_atomic_fetch_add(b_count(p) + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == S - 1;
+    last = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == S - 1;
   __syncthreads();
   if (!last) return;
-  if (threadIdx.x == 0) dev_store32(b_count(p) + tile, 0);  // ready for the next split product
+  if (threadIdx.x == 0) dev_store32(count, 0);  // ready for the next split product
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
     const int e = threadIdx.x + kGT * k;
@@ -567,15 +572,17 @@ __global__ void __launch_bounds__(kGT) k_bx_residual(BatchParams p, const uint16
 
 // w1 / w3 of FFN columns f0 .. f0 + 15 and the SiLU gate (Lfm2MLP.forward,
 // modeling_lfm2.py:135-136): g = bf16(bf16(silu(bf16(w1 . n))) * bf16(w3 . n)).
+template <int MT, bool kFold>
 __global__ void __launch_bounds__(kGT) k_bx_silu(BatchParams p, int l) {
-  __shared__ GemmLdsStaged sh;
-  const int f0 = 16 * blockIdx.x;
+  __shared__ GemmLdsStaged<MT> sh;
+  const int f0 = 16 * blockIdx.x, m0 = 16 * MT * blockIdx.y;
   const uint16_t* wt[2] = {layer_tensor<C_W1, A_W1>(p.weights, l) + (size_t)f0 * kHidden,
                            layer_tensor<C_W3, A_W3>(p.weights, l) + (size_t)f0 * kHidden};
-  gemm_tiles_staged<2, 4>(wt, p, layer_tensor<C_FFNNORM, A_FFNNORM>(p.weights, l), sh);
+  gemm_tiles_staged<2, 4, MT, kFold>(wt, p, layer_tensor<C_FFNNORM, A_FFNNORM>(p.weights, l), sh, m0);
   __syncthreads();
-  uint16_t* g = b_g(p);
-  for (int e = threadIdx.x; e < 16 * p.rows; e += kGT) {
+  uint16_t* g = b_g(p) + (size_t)m0 * kFfn;
+  const int n = 16 * min(p.rows - m0, 16 * MT);
+  for (int e = threadIdx.x; e < n; e += kGT) {
     const int i = e & 15, m = e >> 4;
     const float a = round_bf16(gemm_at<4>(sh, 0, i, m));
     const float b = round_bf16(gemm_at<4>(sh, 1, i, m));
@@ -586,10 +593,12 @@ __global__ void __launch_bounds__(kGT) k_bx_silu(BatchParams p, int l) {
 // q / k / v rows of one head (block b: query head b < 16, key head b - 16,
 // value head b - 24), then per row: q and k through QK-RMSNorm + RoPE at the
 // row's position (norm_rope_lane), k and v appended to the row's sequence
-// cache at that position, q kept for the attention.
+// cache at that position, q kept for the attention. Block (b, y) takes the 16
+// rows from 16 y.
+template <bool kFold>
 __global__ void __launch_bounds__(kGT) k_bx_qkv(BatchParams p, int l) {
-  __shared__ GemmLdsStaged sh;
-  const int b = blockIdx.x;
+  __shared__ GemmLdsStaged<1> sh;
+  const int b = blockIdx.x, m0 = 16 * blockIdx.y, rows = min(p.rows - m0, 16);
   const int row0 = b < 16 ? 64 * b : b < 24 ? kHidden + 64 * (b - 16) : kHidden + 512 + 64 * (b - 24);
   const uint16_t* wq = attn_tensor<A_Q>(p.weights, l) + (size_t)row0 * kHidden;
   const uint16_t* wt[4] = {wq, wq + 16 * kHidden, wq + 32 * kHidden, wq + 48 * kHidden};
@@ -598,7 +607,7 @@ __global__ void __launch_bounds__(kGT) k_bx_qkv(BatchParams p, int l) {
   // norm weights before the weights, the RoPE row once they are requested.
   const float gq = bf16_to_f32(attn_tensor<A_QLN>(p.weights, l)[d]);
   const float gk = bf16_to_f32(attn_tensor<A_KLN>(p.weights, l)[d]);
-  const RowInfo r0 = b_row(p, min(w, p.rows - 1));
+  const RowInfo r0 = b_row(p, m0 + min(w, rows - 1));
   uint16_t cs0 = 0, sn0 = 0;
   const auto rope0 = [&] {
     if (b < 24 && r0.pos >= 0 && r0.pos < p.capacity) {
@@ -606,18 +615,18 @@ __global__ void __launch_bounds__(kGT) k_bx_qkv(BatchParams p, int l) {
       sn0 = p.rope[(size_t)r0.pos * 2 * kHeadDim + kHeadDim + d];
     }
   };
-  gemm_tiles_staged<4, 2>(wt, p, attn_tensor<A_OPNORM>(p.weights, l), sh, rope0);
+  gemm_tiles_staged<4, 2, 1, kFold>(wt, p, attn_tensor<A_OPNORM>(p.weights, l), sh, m0, rope0);
   __syncthreads();
   const int att = l - conv_before(l);
-  for (int m = w; m < p.rows; m += kGW) {
-    const RowInfo r = m == w ? r0 : b_row(p, m);
+  for (int m = w; m < rows; m += kGW) {
+    const RowInfo r = m == w ? r0 : b_row(p, m0 + m);
     if (r.pos < 0 || r.pos >= p.capacity) continue;
     const float raw = round_bf16(gemm_at<2>(sh, d >> 4, d & 15, m));
     if (b < 24) {
       const float cs = bf16_to_f32(m == w ? cs0 : p.rope[(size_t)r.pos * 2 * kHeadDim + d]);
       const float sn = bf16_to_f32(m == w ? sn0 : p.rope[(size_t)r.pos * 2 * kHeadDim + kHeadDim + d]);
       const float o = norm_rope_lane(raw, b < 16 ? gq : gk, cs, sn);
-      if (b < 16) b_q(p)[(size_t)m * kHidden + 64 * b + d] = f32_to_bf16(o);
+      if (b < 16) b_q(p)[(size_t)(m0 + m) * kHidden + 64 * b + d] = f32_to_bf16(o);
       else p.key_cache[kv_head_base(p, r.seq, att, b - 16) + (size_t)r.pos * kHeadDim + d] = f32_to_bf16(o);
     } else {
       p.value_cache[kv_head_base(p, r.seq, att, b - 24) + (size_t)r.pos * kHeadDim + d] = f32_to_bf16(raw);
@@ -682,8 +691,8 @@ __global__ void __launch_bounds__(kGT) k_bx_head(BatchParams p) {
     // the final norm of the batch rows into LDS (RowStage), behind the first
     // round's table rows
     const bool fold = rows <= kFoldRows;
-    RowStage stage;
-    stage.load(fold ? b_x(p) : b_xn(p), final_norm(p.weights), rows, mt);
+    RowStage<kMT> stage;
+    stage.load(fold ? b_x(p) : b_xn(p), final_norm(p.weights), rows, mt, fold);
     load_a(blockIdx.x);
     stage.store(sh.x, sh.ss, mt, fold);
   }
@@ -817,10 +826,10 @@ __global__ void __launch_bounds__(kHidden / 8) k_bx_last_rows(BatchParams p, Pro
 // Y[m][n] = bf16(W[n] . X[m]) for the batch linear test entry point.
 template <int K>
 __global__ void __launch_bounds__(kGT) k_bx_linear(const uint16_t* x, const uint16_t* w, uint16_t* y, int rows, int n) {
-  __shared__ GemmLds sh;
+  __shared__ GemmLds<kMT> sh;
   const int n0 = 16 * blockIdx.x;
   const uint16_t* wt[1] = {w + (size_t)n0 * K};
-  gemm_tiles<1, kGW, K>(wt, x, rows, sh);
+  gemm_tiles<1, kGW, K, kMT>(wt, x, rows, sh);
   __syncthreads();
   for (int e = threadIdx.x; e < 16 * rows; e += kGT) {
     const int i = e & 15, m = e >> 4;
@@ -851,27 +860,48 @@ int launch_pass(const BatchParams& p, bool select, int32_t* tokens_out, uint16_t
   uint16_t* x = reinterpret_cast<uint16_t*>(p.ws + kBwX);
   uint16_t* y = reinterpret_cast<uint16_t*>(p.ws + kBwY);
   uint16_t* xn = reinterpret_cast<uint16_t*>(p.ws + kBwXn);
-  // above kFoldRows rows the norms run once per phase instead of in every
-  // block of the product that reads them
-  const bool fold = p.rows <= kFoldRows;
+  // A product's rows split over blocks in groups of 16 (blocks of one weight
+  // tile land on one XCD, whose L2 then holds it), each forming its rows' norm:
+  // a block that took all 64 rows read 128 KB of activations for 32-128 KB of
+  // weights, on as few as 32 CUs (q|k|v 14.7 us). At 64 rows (four groups)
+  // the gate product would run its norms 640 times: 10.7 us against 9.9 with
+  // the norms in a pass of their own, and the conv 9.2 against 9.0 (two groups
+  // of 32), so there the norms come first. The bits do not depend on it. A
+  // pass of 4 rows 380 -> 337 us, 24 rows 457 -> 412, 48 rows 527 -> 460, 64
+  // rows 571 -> 515.
+  // The conv's window runs along a sequence's rows and its last row
+  // overwrites the state that the first rows read, so its rows are split only
+  // in a decode step, where every row is its own sequence's.
+  const int groups = (p.rows + 15) / 16;
   for (int l = 0; l < kLayers; ++l) {
     const bool attn = is_attn(l);
     const uint16_t* base = p.weights + layer_off(l);
     const uint16_t* op_norm = base + slot_off(attn, attn ? (int)A_OPNORM : (int)C_OPNORM);
     const uint16_t* ffn_norm = base + slot_off(attn, attn ? (int)A_FFNNORM : (int)C_FFNNORM);
-    if (!fold) k_bx_norm<<<p.rows, 2 * kWave, 0, s>>>(p, x, op_norm, xn);
     const uint16_t* w_out = base + slot_off(attn, attn ? (int)A_O : (int)C_OUT);
     const uint16_t* w2 = base + slot_off(attn, attn ? (int)A_W2 : (int)C_W2);
+    const bool fold = groups < kMT, split_conv = groups == 1 || decode_tokens != nullptr;
+    if (!fold || (!attn && !split_conv)) k_bx_norm<<<p.rows, 2 * kWave, 0, s>>>(p, x, op_norm, xn);
     if (attn) {
-      k_bx_qkv<<<32, kGT, 0, s>>>(p, l);
+      if (fold) k_bx_qkv<true><<<dim3(32, groups), kGT, 0, s>>>(p, l);
+      else k_bx_qkv<false><<<dim3(32, groups), kGT, 0, s>>>(p, l);
       k_bx_attention<<<dim3(p.rows, kKvHeads), kAT, 0, s>>>(p, l);
+    } else if (!split_conv) {
+      k_bx_conv<kMT, false><<<kHidden / 8, kGT, 0, s>>>(p, l);
+    } else if (fold) {
+      k_bx_conv<1, true><<<dim3(kHidden / 8, groups), kGT, 0, s>>>(p, l);
     } else {
-      k_bx_conv<<<kHidden / 8, kGT, 0, s>>>(p, l);
+      k_bx_conv<2, false><<<dim3(kHidden / 8, kMT / 2), kGT, 0, s>>>(p, l);
     }
-    k_bx_residual<kHidden, kResSplit><<<kResSplit * kHidden / 16, kGT, 0, s>>>(p, w_out, y);
-    if (!fold) k_bx_norm<<<p.rows, 2 * kWave, 0, s>>>(p, x, ffn_norm, xn);
-    k_bx_silu<<<kFfn / 16, kGT, 0, s>>>(p, l);
-    k_bx_residual<kFfn, kResSplit><<<kResSplit * kHidden / 16, kGT, 0, s>>>(p, w2, b_g_host(p));
+    k_bx_residual<kHidden, kResSplit, 1><<<dim3(kResSplit * kHidden / 16, groups), kGT, 0, s>>>(p, w_out, y);
+    if (fold) {
+      k_bx_silu<1, true><<<dim3(kFfn / 16, groups), kGT, 0, s>>>(p, l);
+    } else {
+      k_bx_norm<<<p.rows, 2 * kWave, 0, s>>>(p, x, ffn_norm, xn);
+      k_bx_silu<kMT, false><<<kFfn / 16, kGT, 0, s>>>(p, l);
+    }
+    if (groups == 1) k_bx_residual<kFfn, kResSplit, 1><<<kResSplit * kHidden / 16, kGT, 0, s>>>(p, w2, b_g_host(p));
+    else k_bx_residual<kFfn, kResSplit, 2><<<dim3(kResSplit * kHidden / 16, (groups + 1) / 2), kGT, 0, s>>>(p, w2, b_g_host(p));
   }
   int rc = check_launch("batch pass");
   if (rc != LFM25_OK) return rc;
