@@ -62,12 +62,12 @@ def run_pass(desc: _lib.Batch, rows: list[tuple[int, int, int]], select: bool, t
 
 
 # Rows from which one sequence's prompt takes a prompt pass (lfm25_prompt_pass)
-# instead of passes of up to MAX_ROWS rows: one pass of 64 rows takes 0.51 ms
+# instead of passes of up to MAX_ROWS rows: one pass of 64 rows takes 0.49 ms
 # and a prompt pass of 64 rows 0.52, of 96 rows 0.57, of 512 rows 0.74.
 PROMPT_ROWS = MAX_ROWS + 1
 # ... and a batch's prompts: up to four passes' rows keep the passes, which
 # give a row the same bits as run_rows does (a prompt pass sums in another
-# order). Four passes of 64 rows take 2.1 ms, a prompt pass of 256 rows 0.64.
+# order). Four passes of 64 rows take 2.0 ms, a prompt pass of 256 rows 0.64.
 BATCH_PROMPT_ROWS = 4 * MAX_ROWS + 1
 
 

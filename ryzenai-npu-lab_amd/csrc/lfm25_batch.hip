@@ -505,8 +505,7 @@ __global__ void __launch_bounds__(kGT) k_bx_conv(BatchParams p, int l) {
 }
 
 // Residual projection of 16 output rows n0 .. n0 + 15: X[m][n] =
-// bf16(X[m][n] + bf16(W[n] . in[m])) (out_proj / o_proj with K = 1024, w2 with
-// K = 2560; the residual add of Lfm2DecoderLayer.forward, modeling_lfm2.py:431).
+// bf16(X[m][n] + bf16(W[n] . in[m])) (w2 with K = 2560; the residual add of Lfm2DecoderLayer.forward, modeling_lfm2.py:431).
 // S blocks per tile and row group (block b: tile b % 64, K slice b / 64), so that S times
 // as many CUs share the weights and, above all, the activations (at 64 rows
 // a tile reads 128-320 KB of them, which one CU's vector cache takes ~10 us
@@ -568,6 +567,65 @@ __global__ void __launch_bounds__(kGT) k_bx_residual(BatchParams p, const uint16
     for (int q = 1; q < S; ++q) sum += __uint_as_float(dev_load32(part + q * kRowsMax * 16 + e));
     x[(size_t)(e >> 4) * kHidden + n0 + (e & 15)] = f32_to_bf16(round_bf16(bf16_to_f32(h[k]) + round_bf16(sum)));
   }
+}
+
+// The same projection for K = 1024 (out_proj / o_proj), a block per tile and
+// group of 16 rows: its waves form all of the tile's chains (kSlices slices of
+// kParts chains, added in the order of k_bx_residual: the same bits), their
+// weights and activations (64 KB) all requested before the first product.
+// Bound by the latency of those loads. At 64 rows 6.5 -> 4.8 us: the exchange
+// through device memory costs more than the sharing gains. (For w2's 160 KB
+// per block it does not: 7.8 us split, 8.5 in one block, and a pass of 16
+// rows, 64 such blocks, 359 -> 406.)
+struct OutShape {
+  static constexpr int K = kHidden;
+  static constexpr int kSlices = kResSplit, kParts = res_ks(K / kResSplit);
+  static constexpr int kSteps = K / (32 * kSlices * kParts);
+  static constexpr int kPer = kSlices * kParts / kGW;  // chains per wave
+  static_assert(kSteps * 32 * kSlices * kParts == K && kPer * kGW == kSlices * kParts, "whole chains per wave");
+};
+__global__ void __launch_bounds__(kGT)
+    k_bx_out(BatchParams p, const uint16_t* w, const uint16_t* in) {
+  using R = OutShape;
+  constexpr int K = R::K;
+  __shared__ f32x4_t part[R::kSlices * R::kParts][kWave];
+  const int t = threadIdx.x, wv = wave_id(), l = lane_id();
+  const int n0 = 16 * blockIdx.x, m0 = 16 * blockIdx.y, rows = min(p.rows - m0, 16);
+  // the element of X that this thread completes, requested before the weights
+  const int m = min(t >> 4, rows - 1), i = t & 15;
+  uint16_t* x = b_x(p) + (size_t)(m0 + m) * kHidden + n0 + i;
+  const uint16_t h = *x;
+  const Rsrc ra = rsrc(w + (size_t)n0 * K, (size_t)16 * K * 2);
+  const Rsrc rb = rsrc(in + (size_t)m0 * K, (size_t)rows * K * 2);  // (rows past `rows` read zeros)
+  const int off = ((l & 15) * K + 8 * (l >> 4)) * 2;
+  bf16x8_t a[R::kPer][R::kSteps], b[R::kPer][R::kSteps];
+#pragma unroll
+  for (int c = 0; c < R::kPer; ++c)
+#pragma unroll
+    for (int st = 0; st < R::kSteps; ++st) {
+      const int col = 32 * ((wv * R::kPer + c) * R::kSteps + st);
+      a[c][st] = load_bf16x8(ra, off, 2 * col);
+      b[c][st] = load_bf16x8(rb, off, 2 * col);
+    }
+#pragma unroll
+  for (int c = 0; c < R::kPer; ++c) {
+    f32x4_t acc{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int st = 0; st < R::kSteps; ++st) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[c][st], b[c][st], acc, 0, 0, 0);
+    part[wv * R::kPer + c][l] = acc;
+  }
+  lds_barrier();
+  if (t >= 16 * rows) return;
+  const int lane = m + 16 * (i >> 2), e = i & 3;
+  float sum = 0.0f;
+#pragma unroll
+  for (int s = 0; s < R::kSlices; ++s) {
+    float v = part[s * R::kParts][lane][e];
+#pragma unroll
+    for (int q = 1; q < R::kParts; ++q) v += part[s * R::kParts + q][lane][e];
+    sum = s == 0 ? v : sum + v;
+  }
+  *x = f32_to_bf16(round_bf16(bf16_to_f32(h) + round_bf16(sum)));
 }
 
 // w1 / w3 of FFN columns f0 .. f0 + 15 and the SiLU gate (Lfm2MLP.forward,
@@ -792,7 +850,7 @@ __global__ void __launch_bounds__(kAT) k_bx_pick(BatchParams p, int blocks, int3
 // call has already cleared and may have flagged)
 __global__ void k_bx_status_clear(BatchParams p, int status) {
   if (threadIdx.x == 0 && status) *b_status(p) = 0;
-  if (threadIdx.x < kHidden / 16) b_count(p)[threadIdx.x] = 0;
+  for (int i = threadIdx.x; i < kMT * kHidden / 16; i += blockDim.x) b_count(p)[i] = 0;
 }
 
 // The host's row table (or decode start positions) into the workspace, from
@@ -868,7 +926,7 @@ int launch_pass(const BatchParams& p, bool select, int32_t* tokens_out, uint16_t
   // the norms in a pass of their own, and the conv 9.2 against 9.0 (two groups
   // of 32), so there the norms come first. The bits do not depend on it. A
   // pass of 4 rows 380 -> 337 us, 24 rows 457 -> 412, 48 rows 527 -> 460, 64
-  // rows 571 -> 515.
+  // rows 571 -> 515 (with k_bx_out 333, 406, 441 and 485).
   // The conv's window runs along a sequence's rows and its last row
   // overwrites the state that the first rows read, so its rows are split only
   // in a decode step, where every row is its own sequence's.
@@ -893,7 +951,7 @@ int launch_pass(const BatchParams& p, bool select, int32_t* tokens_out, uint16_t
     } else {
       k_bx_conv<2, false><<<dim3(kHidden / 8, kMT / 2), kGT, 0, s>>>(p, l);
     }
-    k_bx_residual<kHidden, kResSplit, 1><<<dim3(kResSplit * kHidden / 16, groups), kGT, 0, s>>>(p, w_out, y);
+    k_bx_out<<<dim3(kHidden / 16, groups), kGT, 0, s>>>(p, w_out, y);
     if (fold) {
       k_bx_silu<1, true><<<dim3(kFfn / 16, groups), kGT, 0, s>>>(p, l);
     } else {
