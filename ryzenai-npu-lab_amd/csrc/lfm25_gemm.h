@@ -263,12 +263,13 @@ __device__ __forceinline__ void load_bf16(const uint16_t* p, float (&v)[kN]) {
 // ln(2) times what t's rounding left out; 1 + e^-x is held scaled by
 // 2^-24, so that its reciprocal is a normal number where v_rcp would flush a
 // denormal one. Within 3 units in the last FP32 place, as the form it
-// replaces; infinities and NaN give what that form gave.
+// replaces; infinities and NaN give what that form gave: x itself goes into
+// the exponent, and only what t left out is clamped (it is below 2^-15 where
+// the result is neither 0 nor v, and a NaN at an infinite x).
 __device__ __forceinline__ float over_one_plus_exp(float v, float x) {
   constexpr float kLog2e = 0x1.715476p+0f, kLog2eRest = 0x1.4ae0cp-26f, kLn2 = 0x1.62e43p-1f, kScale = 0x1p-24f;
-  const float c = __builtin_amdgcn_fmed3f(x, -200.0f, 200.0f);  // e^200 scaled is infinity, e^-200 nothing
-  const float t = -c * kLog2e;
-  const float rest = fmaf(-c, kLog2eRest, fmaf(-c, kLog2e, -t));
+  const float t = -x * kLog2e;
+  const float rest = __builtin_amdgcn_fmed3f(fmaf(-x, kLog2eRest, fmaf(-x, kLog2e, -t)), -1.0f, 1.0f);
   const float d = fmaf(__builtin_amdgcn_exp2f(t - 24.0f), fmaf(rest, kLn2, 1.0f), kScale);
   return v * (__builtin_amdgcn_rcpf(d) * kScale);
 }
