@@ -1,6 +1,6 @@
 """The sigmoid gates of csrc/lfm25_gemm.h (over_one_plus_exp), which the
 encoder's Swish, its GLU and the prompt pass's SiLU share: what infinities and
-NaN give where the gated value is not the gate."""
+NaN give where the gated value is not the gate, and the FP32 error."""
 
 from __future__ import annotations
 
@@ -40,3 +40,37 @@ def test_glu_keeps_nan_and_infinities(lab, gpu):
     assert torch.equal(got[~finite & ~torch.isnan(want)], want[~finite & ~torch.isnan(want)])
     # a gate value next to a BF16 boundary may round either way, and the result once more
     assert bool(((got - want).abs()[finite] <= 2.0 ** -7 * want.abs()[finite]).all())
+
+
+def test_sigmoid_error_in_fp32(lab, gpu):
+    """Swish of 3.6 million FP32 numbers (hi + 2^e (lo + lo2) from a product
+    with exact sums, 24 bits each) against 64 bits. The FP32 value is within 7
+    x 2^-24 of the exact one (a unit in the last place each, that is 2 x
+    2^-24, for the exponential and the reciprocal, a rounding each for the
+    correction, the sum and the final product), so the BF16 result is within
+    half a step and that of it."""
+    rows, cols = [], []
+    for e in range(-3, 4):
+        for hi in range(128, 256):
+            rows += [(sign * hi * 2.0 ** (e - 7), 2.0 ** e) for sign in (1, -1)]
+    g = torch.Generator().manual_seed(5)
+    lo2 = torch.randint(0, 256, (2048,), generator=g)
+    a = torch.zeros(len(rows), 64)
+    a[:, :2] = torch.tensor(rows)
+    a[:, 2] = a[:, 1]
+    b = torch.zeros(2048, 64)
+    b[:, 0] = 1
+    b[:, 1] = (torch.arange(2048) % 256) * 2.0 ** -15
+    b[:, 2] = lo2 * 2.0 ** -23
+    ad, bd = a.bfloat16().to(gpu), b.bfloat16().to(gpu)
+    assert torch.equal(ad.cpu().float(), a) and torch.equal(bd.cpu().float(), b)
+    c = torch.empty(len(rows), 2048, dtype=torch.bfloat16, device=gpu)
+    lab._lib.call("lfm25_pk_gemm", ad.data_ptr(), 64, bd.data_ptr(), 64, None, c.data_ptr(), 2048, len(rows), 2048, 64,
+                  2, 1, None, torch.cuda.current_stream().cuda_stream)
+    x = ad.double() @ bd.double().T.contiguous()
+    want = x / (1 + torch.exp(-x))
+    step = torch.ldexp(torch.ones_like(x), torch.frexp(want.abs())[1] - 8)
+    excess = ((c.double() - want).abs() - step / 2) / want.abs() * 2.0 ** 24
+    print(f"largest excess over half a step {float(excess.max()):.2f} x 2^-24, "
+          f"{int((c != want.to(torch.bfloat16)).sum())} values off the nearest")
+    assert float(excess.max()) <= 7
