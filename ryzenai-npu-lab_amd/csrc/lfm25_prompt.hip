@@ -475,7 +475,12 @@ __global__ void __launch_bounds__(kQ * 8) k_pp_attention(Prompt p, PromptRuns ru
 #define LFM25_PP_WAIT(kN) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kN) : "memory")
   copy(0, 0, false);
   copy(1, 1, false);
-  float m = kMasked, z = 0.0f;
+  // m: this lane's largest score so far, mc: m kC rounded, z: the sum of 2^(s
+  // kC - mc). z is scaled only where some lane's maximum grows, by the
+  // difference of the rounded mc that its terms were and will be formed with:
+  // scaled every tile by 2^(m kC - mc), which is not 1 where m did not change,
+  // z was up to 4e-5 off after 64 tiles.
+  float m = kMasked, mc = kMasked * kC, z = 0.0f;
   int stage = 0;
   for (int t = 0; t < tiles; ++t) {
     LFM25_PP_WAIT(kCopies);
@@ -486,19 +491,24 @@ __global__ void __launch_bounds__(kQ * 8) k_pp_attention(Prompt p, PromptRuns ru
     for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
       for (int e = 0; e < 4; ++e) top = fmaxf(top, s[kt][e]);
-    const float next = fmaxf(m, top), mc = next * kC;
+    if (__builtin_amdgcn_ballot_w64(top > m) != 0) {
+      m = fmaxf(m, top);
+      const float next = m * kC;
+      z *= __builtin_amdgcn_exp2f(mc - next);
+      mc = next;
+    }
     float sum = 0.0f;
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
       for (int e = 0; e < 4; ++e) sum += __builtin_amdgcn_exp2f(fmaf(s[kt][e], kC, -mc));
-    z = fmaf(z, __builtin_amdgcn_exp2f(fmaf(m, kC, -mc)), sum);
-    m = next;
+    z += sum;
     stage = stage == 2 ? 0 : stage + 1;
   }
-  const float all = max_groups(m);
-  z = sum_groups(z * __builtin_amdgcn_exp2f((m - all) * kC));
-  const float mc = all * kC, rz = 1.0f / z;
+  const float all = max_groups(m) * kC;
+  z = sum_groups(z * __builtin_amdgcn_exp2f(mc - all));
+  mc = all;
+  const float rz = 1.0f / z;
   // LDS addresses of this lane's value reads: row 4 (l / 16) + (l % 16) / 4 of
   // 16, 8 bytes at dimensions 16 dt + 4 (l % 4) (rows 16 apart keep a_swizzle)
   ValueReads at;
