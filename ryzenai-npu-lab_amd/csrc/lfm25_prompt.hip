@@ -441,7 +441,23 @@ __global__ void __launch_bounds__(kQ * 8) k_pp_attention(Prompt p, PromptRuns ru
     }
   };
   constexpr float kC = 0.125f * 1.44269504088896340736f;
-  constexpr float kMasked = -0x1p99f;  // (a power of two: kMasked * kC is exact, and less itself exactly 0)
+  // The exponent of a score s is s kc - mc, kc = kC and mc = m kC rounded for
+  // the maximum m. What the rounding leaves at s = m is in the sum and in
+  // every probability alike; that it stays in exp2's range too, m kc ends at
+  // kLarge kC (then it is at most 2^3, and the next smaller BF16 score is
+  // still 2^19 below in the exponent). A lane that has seen no key has m =
+  // kNone, below every score.
+  constexpr float kLarge = 0x1p30f, kNone = -0x1.fffffep127f;
+  const auto reference = [&](float m, float& kc, float& mc) {
+    const float a = fabsf(m);
+    kc = a > kLarge ? kC * kLarge / a : kC;
+    mc = m * kc;
+  };
+  // What a sum formed with (m, mc) is scaled by to continue with (to, mc_to):
+  // with maxima 2^22 apart nothing of it is left, and nearer ones have the same kc.
+  const auto rescale = [&](float m, float mc, float to, float mc_to) {
+    return to - m >= 0x1p22f ? 0.0f : __builtin_amdgcn_exp2f(mc - mc_to);
+  };
   // scores of tile t: s[kt][e] = bf16(q . k) of key 64 t + 16 kt + 4 (l / 16) + e
   f32x4 s[4];
   const auto scores = [&](int t, int stage) {
@@ -467,7 +483,7 @@ __global__ void __launch_bounds__(kQ * 8) k_pp_attention(Prompt p, PromptRuns ru
       for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (t * kKeys + 16 * kt + 4 * (l >> 4) + e > pos) s[kt][e] = kMasked;
+          if (t * kKeys + 16 * kt + 4 * (l >> 4) + e > pos) s[kt][e] = -INFINITY;
     }
   };
   // tile t's copies (kN of them per tile and wave) have landed, in every
@@ -475,12 +491,12 @@ __global__ void __launch_bounds__(kQ * 8) k_pp_attention(Prompt p, PromptRuns ru
 #define LFM25_PP_WAIT(kN) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kN) : "memory")
   copy(0, 0, false);
   copy(1, 1, false);
-  // m: this lane's largest score so far, mc: m kC rounded, z: the sum of 2^(s
-  // kC - mc). z is scaled only where some lane's maximum grows, by the
-  // difference of the rounded mc that its terms were and will be formed with:
-  // scaled every tile by 2^(m kC - mc), which is not 1 where m did not change,
-  // z was up to 4e-5 off after 64 tiles.
-  float m = kMasked, mc = kMasked * kC, z = 0.0f;
+  // m: this lane's largest score so far, z: the sum of 2^(s kc - mc), scaled
+  // by the difference of the rounded mc that its terms were and will be formed
+  // with. (Scaled by 2^(m kC - mc), which is not 1 where m did not change, it
+  // was up to 4e-5 off after 64 tiles.)
+  float m = kNone, kc, mc, z = 0.0f;
+  reference(m, kc, mc);
   int stage = 0;
   for (int t = 0; t < tiles; ++t) {
     LFM25_PP_WAIT(kCopies);
@@ -491,23 +507,28 @@ __global__ void __launch_bounds__(kQ * 8) k_pp_attention(Prompt p, PromptRuns ru
     for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
       for (int e = 0; e < 4; ++e) top = fmaxf(top, s[kt][e]);
-    if (__builtin_amdgcn_ballot_w64(top > m) != 0) {
-      m = fmaxf(m, top);
-      const float next = m * kC;
-      z *= __builtin_amdgcn_exp2f(mc - next);
-      mc = next;
+    const float to = fmaxf(m, top), mc0 = mc;
+    kc = kC;
+    mc = to * kC;
+    float f = __builtin_amdgcn_exp2f(mc0 - mc);
+    if (__builtin_amdgcn_ballot_w64(to > kLarge || m < -kLarge) != 0) {  // (rare past the first tile)
+      reference(to, kc, mc);
+      f = rescale(m, mc0, to, mc);
     }
+    m = to;
     float sum = 0.0f;
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) sum += __builtin_amdgcn_exp2f(fmaf(s[kt][e], kC, -mc));
-    z += sum;
+      for (int e = 0; e < 4; ++e) sum += __builtin_amdgcn_exp2f(fmaf(s[kt][e], kc, -mc));
+    z = fmaf(z, f, sum);
     stage = stage == 2 ? 0 : stage + 1;
   }
-  const float all = max_groups(m) * kC;
-  z = sum_groups(z * __builtin_amdgcn_exp2f(mc - all));
-  mc = all;
+  {
+    const float all = max_groups(m), mc0 = mc;
+    reference(all, kc, mc);
+    z = sum_groups(z * rescale(m, mc0, all, mc));
+  }
   const float rz = 1.0f / z;
   // LDS addresses of this lane's value reads: row 4 (l / 16) + (l % 16) / 4 of
   // 16, 8 bytes at dimensions 16 dt + 4 (l % 4) (rows 16 apart keep a_swizzle)
@@ -535,8 +556,8 @@ __global__ void __launch_bounds__(kQ * 8) k_pp_attention(Prompt p, PromptRuns ru
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const f32x4& sk = s[2 * c + i / 2];
-        pw[i] = pack_pair(__builtin_amdgcn_exp2f(fmaf(sk[2 * (i % 2)], kC, -mc)) * rz,
-                      __builtin_amdgcn_exp2f(fmaf(sk[2 * (i % 2) + 1], kC, -mc)) * rz);
+        pw[i] = pack_pair(__builtin_amdgcn_exp2f(fmaf(sk[2 * (i % 2)], kc, -mc)) * rz,
+                      __builtin_amdgcn_exp2f(fmaf(sk[2 * (i % 2) + 1], kc, -mc)) * rz);
       }
       const bf16x8 pf = __builtin_bit_cast(bf16x8, uint4{pw[0], pw[1], pw[2], pw[3]});
       s16x4 v0[4], v1[4];  // V^T: dimension 16 dt + l % 16 of those 8 keys

@@ -45,14 +45,15 @@ def read(bd, s, att, rows) -> np.ndarray:
     return bd.kv(s, att, rows - 1)[1].transpose(1, 0, 2).reshape(rows, A.PICK)
 
 
-@pytest.mark.parametrize("gamma", [2.0])
+@pytest.mark.parametrize("gamma", [2.0, 2.0 ** 55])
 @pytest.mark.parametrize("rows", [70, 1500, 4096])
 def test_uniform_scores(lab, gpu, rows, gamma):
     """Every key the same, in the dimension pair that RoPE leaves alone over
     4,096 positions, so the p of the query at position n - 1 is bf16(1 / n)
-    whatever the scores are (up to +-256 before their scale): the FP32 quotient
-    is within B of 1 / n, B from the sum of n equal terms (15 additions in a
-    tile, one a tile, two over the lanes) and three more roundings."""
+    whatever the scores are (up to +-256 before their scale, or +-2^116): the
+    FP32 quotient is within B of 1 / n, B from the sum of n equal terms (15
+    additions in a tile, one a tile, two over the lanes) and three more
+    roundings."""
     rng = np.random.default_rng(3)
     slow, fast = 31, 5  # a pair of lowest and one of high frequency: k has none of the latter
     c = rng.uniform(0.2, 1.0, (A.TOKENS, A.HEADS)) * rng.choice([-1, 1], (A.TOKENS, A.HEADS))
