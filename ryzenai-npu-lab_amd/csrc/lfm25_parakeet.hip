@@ -604,7 +604,9 @@ __global__ void __launch_bounds__(kAttBlockThreads, 1)
 // T-1-i+j spans for them go from memory straight into MFMA operands, all of a
 // block's loads in flight at once; the values are copied into the wave's LDS
 // and read back transposed. The waves meet for the rows' maxima, and to add
-// their partial values, which are divided by the rows' sums then.
+// their partial values, which are divided by the rows' sums then. The
+// exponentials carry a factor of 1 / 128 (exact), so that the undivided sums
+// overflow no sooner than the values do.
 constexpr int kAkWaves = 4, kAkQueries = 16;
 constexpr int kAkThreads = kAkWaves * kWave;
 constexpr int kAkKeys = kAttT / kAkWaves;    // keys per wave
@@ -644,6 +646,7 @@ __global__ void __launch_bounds__(kAkThreads, 2)
 #if defined(__HIP_DEVICE_COMPILE__)  // (the host pass has no LDS address space)
   __shared__ PkAttKeysLds sh;
   constexpr int kDs = kDk / 32;  // steps of 32 dimensions
+  constexpr float kShare = 1.0f / kAttT;
   const int h = blockIdx.x, b = blockIdx.y, i0 = kAkQueries * blockIdx.z;
   const int t = threadIdx.x, w = wave_id(), l = lane_id(), col = l & 15, g = l >> 4;
   const uint16_t* base = qkv + (size_t)b * kAttT * 3 * kD + h * kDk;
@@ -715,7 +718,7 @@ __global__ void __launch_bounds__(kAkThreads, 2)
   uint32_t hw[4], lw[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const float e0 = expf(s[i / 2][2 * (i % 2)] - top), e1 = expf(s[i / 2][2 * (i % 2) + 1] - top);
+    const float e0 = kShare * expf(s[i / 2][2 * (i % 2)] - top), e1 = kShare * expf(s[i / 2][2 * (i % 2) + 1] - top);
     z += e0 + e1;
     hw[i] = tile::pack_pair(e0, e1);
     lw[i] = tile::pack_pair(e0 - lo_f32(hw[i]), e1 - hi_f32(hw[i]));

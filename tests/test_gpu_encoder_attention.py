@@ -29,3 +29,17 @@ def test_attention_splits(lab, gpu, pk, layer0, batch, valid):  # noqa: F811
         for h in range(8):
             sl = slice(128 * h, 128 * (h + 1))
             assert scale_ulps(got[b][:, sl], want[:, sl]) <= 2.0, (b, h)
+
+
+@pytest.mark.parametrize("batch", [1, 9])
+def test_large_values_do_not_overflow(lab, gpu, batch):
+    """Equal scores over 128 values of 2^122: their mean is 2^122, their sum
+    past FP32's range."""
+    qkv = torch.zeros(batch, T, 3, 1024, dtype=torch.bfloat16, device=gpu)
+    qkv[:, :, 2] = 2.0 ** 122
+    pos = torch.zeros(8, 2 * T, 128, dtype=torch.bfloat16, device=gpu)
+    delta = torch.zeros(8, 128, dtype=torch.bfloat16, device=gpu)
+    out = torch.zeros(batch, T, 1024, dtype=torch.bfloat16, device=gpu)
+    lab._lib.call("lfm25_pk_attention", qkv.data_ptr(), pos.data_ptr(), delta.data_ptr(), out.data_ptr(), batch, T, T,
+                  stream())
+    assert bool((out == 2.0 ** 122).all())
