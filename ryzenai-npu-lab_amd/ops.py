@@ -20,11 +20,16 @@ HIDDEN, FFN, VOCAB = 1024, 2560, 65536
 GAMMA_TILE = 4096  # the reference pads every norm weight to one 64x64 tile
 
 
-def _stream() -> int:
-    """The handle of torch's current stream (0.2 us; the Stream object that
-    torch.cuda.current_stream() makes of it takes 2.8). Asked for after the
-    arguments are known to be GPU tensors, so the device is initialized."""
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+if hasattr(torch._C, "_cuda_getCurrentRawStream") and hasattr(torch._C, "_cuda_getDevice"):
+    def _stream() -> int:
+        """The handle of torch's current stream (0.2 us; the Stream object
+        that torch.cuda.current_stream() makes of it takes 2.8). Asked for
+        after the arguments are known to be GPU tensors, so the device is
+        initialized."""
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+else:  # a torch without these private names
+    def _stream() -> int:
+        return torch.cuda.current_stream().cuda_stream
 
 
 def _check(t: torch.Tensor, name: str, dtype: torch.dtype, numel: int | None = None) -> int:

@@ -5,8 +5,10 @@ same layout as the host), and argument validation of the Python surfaces."""
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import re
 from pathlib import Path
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
@@ -407,3 +409,16 @@ def test_chat_stops_on_eos_and_renders_the_template():
     assert text == "<|startoftext|><|im_start|>user\nhi<|im_end|>\n<|im_start|>assistant\n"
     with pytest.raises(RuntimeError):
         chat.respond([{"role": "user", "content": "hi"}], 4)
+
+
+@pytest.mark.parametrize("name", ["_cuda_getCurrentRawStream", "_cuda_getDevice"])
+def test_stream_handle_without_torchs_private_names(lab, monkeypatch, name):
+    """A torch without the private names that ops asks for the stream: the
+    public call answers."""
+    if hasattr(torch._C, name):
+        monkeypatch.delattr(torch._C, name)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: SimpleNamespace(cuda_stream=77))
+    spec = importlib.util.spec_from_file_location(lab.ops.__package__ + "._ops_again", lab.ops.__file__)
+    ops = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(ops)
+    assert ops._stream() == 77
