@@ -331,12 +331,12 @@ def test_chat_state_reuse_equals_a_fresh_run(lab, model_cls, ck):
 
 
 def test_batched_prefill_matches_the_oracle_and_token_by_token(lab, model_cls, ck):
-    """X8Model.prefill sends a prompt's tokens before the last through
-    matrix-core passes of up to 64 rows (here 70 = 64 + 6): teacher-forced
-    against the oracle the hidden state, conv states and KV rows stay within
-    16 ulps of their scale, the first selected token meets the argmax bar on
-    the GPU's own hidden state, and the following greedy steps stay within
-    the same bounds as the token-by-token prefill."""
+    """X8Model.prefill sends a prompt of more than 64 tokens (here 71) and its
+    selection through one prompt pass: teacher-forced against the oracle the
+    hidden state, conv states and KV rows stay within 16 ulps of their scale,
+    the first selected token meets the argmax bar on the GPU's own hidden
+    state, and the following greedy steps stay within the same bounds as the
+    token-by-token prefill."""
     from parity_helpers import head_pick_check
     prompt = ids(lab, 71, "decode.bprefill")
     m = model_cls(weights=ck, log=lambda *_: None)

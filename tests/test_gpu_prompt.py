@@ -2,7 +2,9 @@
 (lfm25_batch_pass, which the oracle holds elsewhere) on the same rows: both
 round at the same points and sum in different FP32 orders, so hidden states,
 conv states and KV rows agree within the bound that holds each of them to the
-oracle, twice (16 BF16 ulps of the vector's scale each)."""
+oracle, twice (16 BF16 ulps of the vector's scale each), and in the 2-norm
+within what the roundings of the layers before them give (drift). The
+attention and the conv gate alone, row by row: test_gpu_prompt_stages.py."""
 
 from __future__ import annotations
 
@@ -30,6 +32,21 @@ def ck(lab):
 def scale_ulps(got, want) -> float:
     s = float(np.max(np.abs(want)))
     return float(np.max(np.abs(got - want))) / 2.0 ** (np.floor(np.log2(s)) - 7) if s > 0 else float(np.max(np.abs(got)))
+
+
+def rel(got, want, axis=None):
+    """Relative error in the 2-norm, of the whole or along an axis."""
+    return np.sqrt(np.sum(np.square(got - want), axis) / np.sum(np.square(want), axis))
+
+
+def drift(layers: int) -> float:
+    """What two orders of sums differ by (2-norm, relative) after `layers`
+    layers: where the inputs of a BF16 rounding differ, its errors are
+    independent, 2^-9 / sqrt(3) each on either side, and a layer chains about
+    eight (norms, projections, gates, residuals), so 4.5e-3 a layer, adding up
+    as squares. (Measured 0.7 to 1.8 times that; a first layer has only the
+    values next to a boundary, less than one.)"""
+    return 4.5e-3 * max(layers, 1) ** 0.5
 
 
 def by_passes(bd, runs, ids):
@@ -72,20 +89,28 @@ def test_prompt_pass_matches_the_batched_pass(lab, gpu, batch, ck, capacity, bef
         g = np.random.default_rng(7)
         for s, n in before.items():
             by_passes(bd, [(s, 0, n)], [g.integers(0, VOCAB, n)])
-        # rows past the prompts' ends hold junk: none of it may be read
-        bd.keys.view(3, 6, 8, capacity, 64)[:, :, :, -1] = float("nan") if capacity == 64 else 0
+    # every cache row of the prompt pass's decoder that is not a sequence's yet
+    # holds a NaN: none of it may be read
+    for cache in (b.keys, b.values):
+        for s in range(3):
+            cache.view(3, 6, 8, capacity, 64)[s, :, :, before.get(s, 0):] = float("nan")
     ids = [rng.integers(0, VOCAB, n) for _, _, n in runs]
     want = by_passes(a, runs, ids)
     got, tok = by_prompt_pass(lab, b, runs, ids, gpu)
     assert scale_ulps(got, want) <= 32
+    assert max(rel(x, y) for x, y in zip(got, want)) <= 2.5 * drift(14)
+    kinds = lab.weights.KINDS
+    conv_layers, attn_layers = ([i for i, k in enumerate(kinds) if k == kind] for kind in ("conv", "attention"))
     table = torch.from_numpy(ck["model.embed_tokens.weight"].view(np.int16)).to(gpu).view(torch.bfloat16).double()
     gamma = torch.from_numpy(ck["model.embedding_norm.weight"].view(np.int16)).to(gpu).view(torch.bfloat16).double()
     for r, (s, pos, n) in enumerate(runs):
         for c in range(8):
             assert scale_ulps(b.conv_state(s, c), a.conv_state(s, c)) <= 32, (s, c)
+            assert rel(b.conv_state(s, c), a.conv_state(s, c)) <= 2.5 * drift(conv_layers[c]), (s, c)
         for l in range(6):
             for x, y in zip(b.kv(s, l, pos + n - 1), a.kv(s, l, pos + n - 1)):
                 assert scale_ulps(x, y) <= 32, (s, l)
+                assert rel(x, y, -1).max() <= 3.5 * drift(attn_layers[l]), (s, l)  # each row of 64 by itself
         # the selection is a maximum of its own hidden state's logits, within a BF16 step
         x = torch.from_numpy(got[r]).to(gpu).double()
         logits = table @ (x / torch.sqrt((x * x).mean() + 1e-5) * gamma)
@@ -115,3 +140,33 @@ def test_prompt_pass_rejects_bad_runs(lab, gpu, batch, ck):
         with pytest.raises(ValueError):
             lab._lib.call("lfm25_prompt_pass", bd._desc, ids.data_ptr(), table.ctypes.data, len(runs), None, None,
                           ws.data_ptr(), torch.cuda.current_stream().cuda_stream)
+
+
+@pytest.mark.parametrize("most,lengths,before", [
+    (100, (130, 90, 70), (0, 5, 0)),      # prompts cut at 100 rows, one of them twice
+    (129, (258, 1, 64), (0, 0, 33)),      # whole passes of one prompt, and the rest in the third
+    (4096, (2060, 1990, 60), (3, 0, 0)),  # the real limit, 4,110 rows
+])
+def test_batch_prefill_cuts_prompts_at_the_passes_limit(lab, gpu, batch, ck, monkeypatch, most, lengths, before):
+    """BatchDecoder.prefill over more rows than a prompt pass takes: a prompt
+    goes on in the next pass where the last one cut it, on its cached keys and
+    its conv state, so states, caches, positions and next tokens are the bits
+    of a pass per prompt (a run's bits do not depend on the runs beside it)."""
+    capacity = max(n + p for n, p in zip(lengths, before)) + 1
+    a = batch.BatchDecoder(3, capacity, weights=ck)
+    b = batch.BatchDecoder(3, capacity, share=a)
+    prompts = [[int(t) for t in np.random.default_rng(s).integers(0, VOCAB, n)] for s, n in enumerate(lengths)]
+    for bd in (a, b):
+        for s, n in enumerate(before):
+            if n:
+                by_passes(bd, [(s, 0, n)], [np.arange(n)])
+    want = [int(by_prompt_pass(lab, a, [(s, before[s], len(p))], [np.asarray(p)], gpu)[1][0])
+            for s, p in enumerate(prompts)]
+    passes, whole = [], batch.run_prompt
+    monkeypatch.setattr(batch, "run_prompt", lambda d, w, t, runs, *rest: (passes.append(runs), whole(d, w, t, runs, *rest)))
+    monkeypatch.setattr(lab._lib, "PROMPT_MAX_ROWS", most)
+    assert b.prefill(prompts) == want
+    assert b.positions == [n + p for n, p in zip(lengths, before)]
+    assert len(passes) == -(-sum(lengths) // most) and all(sum(r[2] for r in runs) <= most for runs in passes)
+    for mine, theirs in ((b.conv_states, a.conv_states), (b.keys, a.keys), (b.values, a.values)):
+        assert torch.equal(mine.view(torch.int16), theirs.view(torch.int16))

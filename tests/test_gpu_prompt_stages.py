@@ -1,5 +1,7 @@
-"""The prompt pass's attention alone (attention_probe.py's weights), with every
-cache row that the pass has not written a NaN."""
+"""The prompt pass's attention and gated conv alone (attention_probe.py's
+weights), every row against the oracle: at the edges of query and key tiles,
+across runs and earlier positions, with every cache row that the pass has not
+written a NaN."""
 
 from __future__ import annotations
 
@@ -10,10 +12,13 @@ import pytest
 import torch
 
 import attention_probe as A
+from oracle import lfm25 as O
+from parity_helpers import attention_interval
 
 pytestmark = pytest.mark.gpu
 
 U = 2.0 ** -24
+EDGES = (0, 1, 15, 16, 31, 32, 63)  # of the query tiles
 
 
 def decoder(capacity, ck):
@@ -45,6 +50,44 @@ def read(bd, s, att, rows) -> np.ndarray:
     return bd.kv(s, att, rows - 1)[1].transpose(1, 0, 2).reshape(rows, A.PICK)
 
 
+# ------------------------------------------------------------------ attention
+
+
+@pytest.mark.parametrize("capacity,before,runs", [
+    (64, {}, [(0, 0, 1)]),
+    (96, {0: 3, 1: 1}, [(1, 1, 16), (0, 3, 17), (2, 0, 15)]),   # around a 16-query tile
+    (256, {0: 62}, [(2, 0, 63), (0, 62, 3), (1, 0, 65)]),       # key counts 63, 64, 65 both ways
+    (300, {2: 64}, [(2, 64, 129), (1, 0, 64), (0, 0, 2)]),
+    (1100, {1: 7}, [(0, 0, 1031), (1, 7, 33)]),                 # 32 queries a block
+    (2200, {1: 100}, [(1, 100, 2050), (0, 0, 31)]),             # 64 queries a block
+])
+def test_attention_rows(lab, gpu, capacity, before, runs):
+    rng = np.random.default_rng(capacity)
+    sign = lambda heads: rng.choice([-1.0, 1.0], (A.TOKENS, heads, A.DIM))  # noqa: E731
+    q, k, v = sign(A.HEADS), sign(A.KV_HEADS), A.bf(rng.standard_normal((A.TOKENS, A.KV_HEADS, A.DIM)) / 128)
+    gq, gk = np.full(A.DIM, 2.0), np.ones(A.DIM)
+    bd = decoder(capacity, A.attention_checkpoint(lab, q, k, v, gq, gk))
+    tokens = rng.integers(0, A.TOKENS, (3, capacity))
+    run(lab, bd, before, runs, tokens, gpu)
+    for s, pos, n in runs:
+        end = pos + n
+        ids = tokens[s][:end]
+        keys, values = bd.kv(s, 0, end - 1)
+        kr = A.norm_rope(k[ids], gk, np.arange(end)).transpose(1, 0, 2)
+        assert np.array_equal(keys, kr) and np.array_equal(values, v[ids].transpose(1, 0, 2))
+        got = read(bd, s, 1, end)
+        rows = {p for p in range(pos, end) if n <= 70 or (p - pos) // 64 % 4 == 0 and (p - pos) % 64 in EDGES}
+        rows |= {p for p in range(pos, end) if p >= end - 2 or p in (63, 64, 65, 127, 128)}
+        qr = A.norm_rope(q[ids], gq, np.arange(end))
+        for p in sorted(rows):
+            # FP32 roundings on one path: the sum of the probabilities takes a
+            # lane's 16 per tile, a tile at a time, then the four lanes; the
+            # context 32 keys a product
+            lo, hi = attention_interval(qr[p], kr[:, :p + 1], values[:, :p + 1], 64 + (p + 1) // 32)
+            inside = (got[p] >= lo[A.picked()]) & (got[p] <= hi[A.picked()])
+            assert inside.all(), (s, p, np.flatnonzero(~inside)[:4], got[p][~inside][:4])
+
+
 @pytest.mark.parametrize("gamma", [2.0, 2.0 ** 55])
 @pytest.mark.parametrize("rows", [70, 1500, 4096])
 def test_uniform_scores(lab, gpu, rows, gamma):
@@ -73,3 +116,38 @@ def test_uniform_scores(lab, gpu, rows, gamma):
     bad = ~((got >= lo) & (got <= hi))
     i, j = np.argwhere(bad)[0] if bad.any() else (0, 0)
     assert not bad.any(), (int(bad.any(axis=1).sum()), int(n[i, 0]), j, float(got[i, j]), float(lo[i, 0]), float(hi[i, 0]))
+
+
+# ------------------------------------------------------------------ gated conv
+
+
+@pytest.mark.parametrize("before,runs", [
+    ({}, [(0, 0, 1)]),
+    ({0: 3, 2: 1}, [(1, 0, 2), (0, 3, 1), (2, 1, 3)]),       # runs of one, two and three rows
+    ({1: 2}, [(2, 0, 4), (1, 2, 2), (0, 0, 70)]),
+    ({1: 65}, [(1, 65, 1), (0, 0, 2), (2, 0, 301)]),
+])
+def test_conv_rows(lab, gpu, before, runs):
+    """Layer 0's conv gate, bit for bit (the oracle rounds at the same points
+    and every sum is exact or in the same order), and the state it leaves."""
+    rng = np.random.default_rng(len(runs))
+    b, x = (A.bf(rng.standard_normal((A.TOKENS, A.HIDDEN)) / 2) for _ in range(2))
+    c = A.bf(rng.standard_normal((A.TOKENS, A.HIDDEN)) / 128)
+    taps = A.bf(rng.standard_normal((A.HIDDEN, 3)) / 2)
+    ck = A.checkpoint(lab)
+    ck["model.layers.0.conv.in_proj.weight"] = A.columns(np.concatenate([b, c, x], axis=1))
+    ck["model.layers.0.conv.conv.weight"] = A.bits(taps).reshape(A.HIDDEN, 1, 3)
+    out = np.zeros((A.HIDDEN, A.HIDDEN), np.uint16)
+    out[np.arange(A.PICK), 2 * np.arange(A.PICK)] = A.bits(1.0)
+    ck["model.layers.0.conv.out_proj.weight"] = out
+    A.read_back(ck, 2)
+    bd = decoder(400, ck)
+    tokens = rng.integers(0, A.TOKENS, (3, 400))
+    run(lab, bd, before, runs, tokens, gpu)
+    for s, pos, n in runs:
+        state, want = np.zeros((A.HIDDEN, 3), np.float32), []
+        for t in tokens[s][:pos + n]:
+            y, state = O.conv_gate(b[t], c[t], x[t], taps, state)
+            want.append(y[::2])
+        assert np.array_equal(read(bd, s, 0, pos + n), np.stack(want)), s
+        assert np.array_equal(bd.conv_state(s, 0), state), s
