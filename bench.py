@@ -427,16 +427,14 @@ def main_encoder(args, lab):
     return 0
 
 
-PREFILL_ROWS = 64  # prompt positions per matrix-core pass
-
-
 def main_prefill(args, lab):
     """Time to first token of a `--prompt P` prompt, as X8Model.prefill runs it:
-    the P - 1 tokens before the last in matrix-core passes of up to 64 rows
-    (lfm25_batch_pass on the decoder's caches), then one decode step that
-    consumes the last token and selects the first reply token. Also timed:
-    the same prompt token by token through the persistent decode. Each
-    variant runs once untimed, then `--steps` times from a reset state."""
+    the prompt and the selection of the first reply token in one matrix-core
+    pass on the decoder's caches (lfm25_prompt_pass, up to 64 tokens
+    lfm25_batch_pass; up to 4 tokens one decode call), then the position that
+    a decode continues from. Also timed: the same prompt token by token
+    through the persistent decode. Each variant runs once untimed, then
+    `--steps` times from a reset state."""
     import ctypes
     import numpy as np
     hip = importlib.import_module("ryzenai-npu-lab_amd.hip")
@@ -458,27 +456,32 @@ def main_prefill(args, lab):
         "workspace": hip.Buffer.zeros(lib.lfm25_decoder_workspace_bytes()),
         "batch_ws": hip.Buffer.zeros(lib.lfm25_batch_workspace_bytes()),
         "tokens_in": hip.Buffer.from_array(np.asarray(prompt, np.int32)),
-        "last": hip.Buffer.from_array(np.asarray(prompt[-1:], np.int32)),
-        "tokens_out": hip.Buffer(64),
+        "tokens_out": hip.Buffer(4 * lab._lib.BATCH_MAX_ROWS),
+        "hidden": hip.Buffer(lab._lib.BATCH_MAX_ROWS * W.HIDDEN * 2),
+        "prompt_ws": hip.Buffer(lib.lfm25_prompt_workspace_bytes(P)),
     }
     b = {k: v.ptr for k, v in bufs.items()}
     desc = lab._lib.Decoder(b["weights"], b["embedding"], b["rope"], b["conv"], b["keys"], b["values"],
                             b["workspace"], cap, int(table.shape[0]))
     batch = lab._lib.Batch(b["weights"], b["embedding"], b["rope"], b["conv"], b["keys"], b["values"],
                            b["batch_ws"], 1, cap, int(table.shape[0]))
-    ctl = np.zeros(1, np.int32)
-    tables = []
-    for start in range(0, P - 1, PREFILL_ROWS):
-        chunk = prompt[start:min(start + PREFILL_ROWS, P - 1)]
-        tables.append(np.asarray([(t, 0, start + i) for i, t in enumerate(chunk)], np.int32))
+    few, rows_most = 4, lab._lib.BATCH_MAX_ROWS  # model.PB and PROMPT_ROWS - 1 (that module would load torch)
+    ctl = np.asarray([P], np.int32)
+    runs = np.asarray([(0, 0, P)], np.int32)
+    rows = np.asarray([(t, 0, i) for i, t in enumerate(prompt)], np.int32)
+    entry = "lfm25_decode" if P <= few else "lfm25_batch_pass" if P <= rows_most else "lfm25_prompt_pass"
 
     def batched():
+        if P <= few:
+            return token_by_token()
         lab._lib.call("lfm25_decoder_reset", desc, None)
-        for rows in tables:
-            lab._lib.call("lfm25_batch_pass", ctypes.byref(batch), rows.ctypes.data, len(rows), 0, None, None, None)
-        ctl[0] = P - 1
+        if P <= rows_most:
+            lab._lib.call("lfm25_batch_pass", ctypes.byref(batch), rows.ctypes.data, P, 1, b["tokens_out"],
+                          b["hidden"], None)
+        else:
+            lab._lib.call("lfm25_prompt_pass", ctypes.byref(batch), b["tokens_in"], runs.ctypes.data, 1,
+                          b["tokens_out"], b["hidden"], b["prompt_ws"], None)
         bufs["workspace"].upload(ctl)  # the position the decode continues from (host-ordered: a blocking copy)
-        lab._lib.call("lfm25_decode", desc, b["last"], 1, 1, b["tokens_out"], lab._lib.EXEC_PERSISTENT, None)
 
     def token_by_token():
         lab._lib.call("lfm25_decoder_reset", desc, None)
@@ -502,7 +505,8 @@ def main_prefill(args, lab):
         if status:
             print(f"prefill ({name}) status 0x{status:x}", file=sys.stderr)
             return 1
-        tok = int(bufs["tokens_out"].download(np.int32, 1)[0])
+        last = P - 1 if name == "batched" and entry == "lfm25_batch_pass" else 0  # (a batched pass selects for every row)
+        tok = int(bufs["tokens_out"].download(np.int32, last + 1)[last])
         ev = sorted(t[0] for t in times)
         wall = sorted(t[1] for t in times)
         results[name] = {"ms": ev[len(ev) // 2], "wall_ms": wall[len(wall) // 2], "first_token": tok}
@@ -512,9 +516,8 @@ def main_prefill(args, lab):
         "value": round(ms, 3), "unit": "ms", "n_gpus": 1, "steps": args.steps, "warmup": 1,
         "ms_per_step": round(ms, 4), "higher_is_better": False, "scaling": "weak", "vs_baseline": None,
         "dtype": "bf16", "data": "synthetic (random-init N(0,0.02) weights, uniform prompt ids, seed 0)",
-        "config": {"workload": f"prompt of {P} uniform ids: {P - 1} in matrix-core passes of up to "
-                               f"{PREFILL_ROWS} rows, the last in one decode step that selects the first token",
-                   "prompt": P, "passes": len(tables)},
+        "config": {"workload": f"prompt of {P} uniform ids and the selection of the first token in one {entry}",
+                   "prompt": P, "passes": 1},
         "prompt_tok_s": round(P / (ms * 1e-3), 1),
         "token_by_token_ms": round(results["token_by_token"]["ms"], 3),
         "first_tokens": [results["batched"]["first_token"], results["token_by_token"]["first_token"]],
