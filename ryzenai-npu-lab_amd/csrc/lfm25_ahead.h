@@ -1,8 +1,8 @@
-// Reading the next product's weights ahead, into L2.
+// Reading the next product's weights ahead, out of HBM.
 //
 // A product of few rows is bound by its weights' way from HBM: its blocks
 // start with nothing and the first bytes take 2-3 us (128 x 4096 x 1024 takes
-// 4.8 us with its weights in L2 and 7.4 with them in HBM), while HBM idles
+// 4.8 us with its weights cached and 7.4 with them in HBM), while HBM idles
 // most of the time. So a product carries extra blocks that touch each
 // 128-byte line of the weights that the products after it will read. (Extra
 // blocks in the short passes between products, norms and gates, made those
@@ -12,7 +12,9 @@
 // that the product's blocks on XCD x will read. (Where a block does not land
 // on XCD blockIdx % 8 nothing but the gain is lost.) Measured: a prompt pass
 // of 250 rows 718 -> 644 us, of 64 rows 619 -> 523, of 4 rows 585 -> 486; one
-// encoder window 173 -> 170, sixteen 410 -> 398.
+// encoder window 173 -> 170. (How much of it L2 gives and how much the
+// memory-side cache behind it is not known: counters of single kernels show
+// the lines fetched anew past L2.)
 #pragma once
 #include "lfm25_device.h"
 
