@@ -3,7 +3,7 @@
 // as four kernels per block phase kind, one stream:
 //
 //   GEMM      C = bf16(epi(A . B + bias)) on the matrix cores, 32 x 64 to
-//             128 x 128 block tiles (lfm25_gemm.h; replaces gemm_step / pk_wx /
+//             256 x 128 block tiles (lfm25_gemm.h; replaces gemm_step / pk_wx /
 //             epilogue, pk_fast.cc:167-231, pk_core.cc:169-183)
 //   LN        scaled residual + LayerNorm (+ a second LayerNorm)
 //             (layer_norm / residual / ln_frame, pk_core.cc:55-116)
@@ -59,7 +59,8 @@ __device__ __forceinline__ float max_lanes16(float v) {
 // ------------------------------------------------------------------ GEMM
 
 // C[m][n] = bf16(epi(sum_k A[m][k] Bt[n][k] + bias[n])), one block tile per
-// block (lfm25_gemm.h; blockIdx.x: tile, blockIdx.y: K split). EPI_RESIDUAL: C = bf16(C + scale bf16(sum)), C the residual stream.
+// block (lfm25_gemm.h; blockIdx.x: tile, blockIdx.y: K split). EPI_RESIDUAL:
+// C = bf16(C + scale bf16(sum)), C the residual stream.
 //
 // Split K (kSplit): block z covers K range [z * kchunk, (z + 1) * kchunk) and
 // writes its FP32 partial tile to part[z][M][N]; k_pk_splitk or
@@ -176,7 +177,7 @@ __device__ __forceinline__ void sum_partials(f32x4_t (&y)[NQ], const float* p, s
   for (int z = 0; z < splits; z += G) add_partials<G>(y, p, stride, z, splits);
 }
 // Partials per round trip for `splits` of them: the next power of two, at
-// most 8 (a one-window product has 8 splits).
+// most 8 (lfm25_pk_gemm's callers name any; the encoder's have 2 or 4).
 inline int partial_group(int splits) { return splits <= 1 ? 1 : splits <= 2 ? 2 : splits <= 4 ? 4 : 8; }
 
 // Sum of the `splits` FP32 partial products in index order (G of them per

@@ -286,10 +286,9 @@ def test_one_layer_matches_mirror(pk, gpu, layer0):
 
 @pytest.mark.parametrize("batch,check", [(16, (0, 13)), (3, (0, 1, 2))])
 def test_batch_matches_mirror(pk, gpu, layer0, batch, check):
-    """Sixteen windows: the wide products run on 256-row tiles, the d-wide
-    ones in 2 K splits. Three windows: 384 rows, so the residual + LayerNorm
-    reductions take the many-row form with 8 and 16 K splits, summed two
-    partials per round trip."""
+    """Sixteen windows: the wide products run on 256-row tiles. Three windows:
+    384 rows on 32 x 64 tiles. In both the d-wide products are whole along K
+    and add the residual in their epilogue."""
     enc = pk.PkEncoder(layers=[layer0])
     x = _inputs(batch, 55)
     valid = 125
