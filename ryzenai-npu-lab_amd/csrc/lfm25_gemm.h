@@ -89,6 +89,26 @@ __device__ __forceinline__ void copy_offsets(Copies<S>& c, int lda, int ldb, con
   }
 }
 
+// The same as 64-bit addresses, where rows lie farther apart than 32-bit
+// offsets reach. Rows past `rows` repeat the last one.
+template <typename S>
+struct FarRows {
+  const uint16_t *a[S::kAI], *b[S::kBI];
+  __device__ __forceinline__ FarRows(const uint16_t* a_base, size_t lda, int rows, const uint16_t* b_base, size_t ldb) {
+    const int w = wave_id(), l = lane_id();
+#pragma unroll
+    for (int i = 0; i < S::kAI; ++i) {
+      const int p = (S::kAI * w + i) * kWave + l, r = p / kChunks, q = (p % kChunks) ^ a_swizzle(r);
+      a[i] = a_base + min(r, rows - 1) * lda + 8 * q;
+    }
+#pragma unroll
+    for (int i = 0; i < S::kBI; ++i) {
+      const int p = (S::kBI * w + i) * kWave + l, r = p / kChunks, q = (p % kChunks) ^ b_swizzle<S>(r);
+      b[i] = b_base + r * ldb + 8 * q;
+    }
+  }
+};
+
 // A wave's results: v[nt][mt][e] is C at row m = 16 (kMT wm + mt) + l % 16 and
 // column n = 16 kNT wn + kLaneN (l / 16) + 4 nt + e of the block tile.
 template <typename S>
@@ -128,16 +148,30 @@ __device__ __forceinline__ void interleave() {
 // acc += the block tile's product over `steps` K steps. The
 // descriptors cover the tile's rows inside the matrix (a lane offset past
 // them touches no memory, and what its row's products are is not used; the
-// step's offset is scalar and not checked). Leaves no copy in flight.
-template <typename S>
+// step's offset is scalar and not checked). Or (kFar) all of it from `far`.
+// Leaves no copy in flight.
+template <typename S, bool kFar = false>
 __device__ __forceinline__ void product(Lds<S>& sh, const void* a_base, uint32_t a_bytes, const void* b_base,
-                                        uint32_t b_bytes, const Copies<S>& c, int steps, Acc<S>& acc) {
+                                        uint32_t b_bytes, const Copies<S>& c, int steps, Acc<S>& acc,
+                                        const FarRows<S>* far = nullptr) {
 #if defined(__HIP_DEVICE_COMPILE__)  // (the host pass has no LDS address space)
   const int w = wave_id(), l = lane_id();
   const int wm = w % S::kWM, wn = w / S::kWM;
   // steps past the last copy nothing: an empty descriptor, so that every
-  // step leaves the same number of loads to count
+  // step leaves the same number of loads to count (far rows: the last step
+  // again, into a stage that nothing reads)
   const auto copy = [&](int step, int stage) {
+    if constexpr (kFar) {
+      typedef __attribute__((address_space(1))) void GlobalVoid;
+      const int k = min(step, steps - 1) * kStep;
+#pragma unroll
+      for (int i = 0; i < S::kAI; ++i)
+        __builtin_amdgcn_global_load_lds((GlobalVoid*)(far->a[i] + k), (LdsVoid*)&sh.a[stage][(S::kAI * w + i) * kWave], 16, 0, 0);
+#pragma unroll
+      for (int i = 0; i < S::kBI; ++i)
+        __builtin_amdgcn_global_load_lds((GlobalVoid*)(far->b[i] + k), (LdsVoid*)&sh.b[stage][(S::kBI * w + i) * kWave], 16, 0, 0);
+      return;
+    }
     const bool in = step < steps;
     const Rsrc ra = make_rsrc(a_base, in ? a_bytes : 0), rb = make_rsrc(b_base, in ? b_bytes : 0);
     const int k = in ? step * kStep * 2 : 0;
@@ -195,7 +229,7 @@ __device__ __forceinline__ void product(Lds<S>& sh, const void* a_base, uint32_t
     interleave<S, kPer>();
     stage = next;
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the empty copies' LDS writes, before the block's LDS is given back
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last copies' LDS writes, before the block's LDS is given back
 #endif
 }
 

@@ -91,7 +91,7 @@ __device__ __forceinline__ float epilogue(float v, float b) {
   return v;
 }
 
-template <int EPI, bool kSplit, typename S>
+template <int EPI, bool kSplit, bool kFar, typename S>
 __global__ void __launch_bounds__(S::kThreads, 2) k_pk_gemm(const PkGemm g) {
   extern __shared__ __attribute__((aligned(16))) char lds_raw[];
   auto& sh = *reinterpret_cast<tile::Lds<S>*>(lds_raw);
@@ -102,13 +102,20 @@ __global__ void __launch_bounds__(S::kThreads, 2) k_pk_gemm(const PkGemm g) {
   const int n0 = tn * S::kTN, m0 = tm * S::kTM, z = blockIdx.y;
   const size_t kbeg = kSplit ? (size_t)z * g.kchunk : 0;
   tile::Copies<S> at;
-  tile::copy_offsets<S>(at, g.lda, g.ldb, [](int r) { return r; });
   tile::Acc<S> acc;
-  acc.zero();
-  // a descriptor ends with the last row's last K element of this block's range
-  tile::product<S>(sh, g.A + (size_t)m0 * g.lda + kbeg,
-                   ((uint32_t)(min(S::kTM, g.M - m0) - 1) * g.lda + g.kchunk) * 2, g.Bt + (size_t)n0 * g.ldb + kbeg,
-                   ((uint32_t)(S::kTN - 1) * g.ldb + g.kchunk) * 2, at, g.kchunk / kBK, acc);
+  if constexpr (kFar) {
+    const tile::FarRows<S> far(g.A + (size_t)m0 * g.lda + kbeg, g.lda, min(S::kTM, g.M - m0),
+                               g.Bt + (size_t)n0 * g.ldb + kbeg, g.ldb);
+    acc.zero();
+    tile::product<S, true>(sh, nullptr, 0, nullptr, 0, at, g.kchunk / kBK, acc, &far);
+  } else {
+    tile::copy_offsets<S>(at, g.lda, g.ldb, [](int r) { return r; });
+    acc.zero();
+    // a descriptor ends with the last row's last K element of this block's range
+    tile::product<S>(sh, g.A + (size_t)m0 * g.lda + kbeg,
+                     ((uint32_t)(min(S::kTM, g.M - m0) - 1) * g.lda + g.kchunk) * 2, g.Bt + (size_t)n0 * g.ldb + kbeg,
+                     ((uint32_t)(S::kTN - 1) * g.ldb + g.kchunk) * 2, at, g.kchunk / kBK, acc);
+  }
   tile::each_row<S>(acc, m0, n0, g.M, [&](int m, int n, float (&v)[S::kLaneN]) {
     if constexpr (kSplit) {
       f32x4_t* p = reinterpret_cast<f32x4_t*>(g.part + ((size_t)z * g.M + m) * g.N + n);
@@ -128,19 +135,6 @@ __global__ void __launch_bounds__(S::kThreads, 2) k_pk_gemm(const PkGemm g) {
       tile::store_bf16<S::kLaneN>(c, v, g.wide);
     }
   });
-}
-
-// The same product where rows lie farther apart than a tile's 32-bit offsets
-// reach (kFarRows elements): an output per thread, 64-bit addresses.
-constexpr int kFarRows = 1 << 22;
-template <int EPI>
-__global__ void __launch_bounds__(256) k_pk_gemm_far(const PkGemm g) {
-  const int n = blockIdx.x * 256 + threadIdx.x, m = blockIdx.y;
-  if (n >= g.N) return;
-  const uint16_t *a = g.A + (size_t)m * g.lda, *b = g.Bt + (size_t)n * g.ldb;
-  float acc = 0.0f;
-  for (int k = 0; k < g.kchunk; ++k) acc = fmaf(bf16_to_f32(a[k]), bf16_to_f32(b[k]), acc);
-  g.C[(size_t)m * g.ldc + n] = f32_to_bf16(epilogue<EPI>(acc, EPI == EPI_BIAS ? bf16_to_f32(g.bias[n]) : 0.0f));
 }
 
 // y += partials z .. z + G - 1 of a thread's NQ x 4 values (partial i at
@@ -880,15 +874,26 @@ int pick_splits(int m, int n, int k) {
   return splits;
 }
 
+template <int EPI, bool kSplit, bool kFar, typename S>
+void launch_tiles(PkGemm g, int splits, hipStream_t s) {
+  g.tiles = tile::tiles_of<S>(g.M, g.N, (int64_t)g.M * g.kchunk * 2);
+  const int blocks = ahead_blocks(g.ahead, g.tiles.blocks(), S::kThreads);
+  k_pk_gemm<EPI, kSplit, kFar, S><<<dim3(blocks, splits), S::kThreads, sizeof(tile::Lds<S>), s>>>(g);
+}
 template <int EPI, bool kSplit>
 void launch_gemm(const PkGemm& g, int splits, hipStream_t s) {
-  tile::with_shape(g.M, g.N, splits, [&](auto shape) {
-    using S = decltype(shape);
-    PkGemm h = g;
-    h.tiles = tile::tiles_of<S>(g.M, g.N, (int64_t)g.M * g.kchunk * 2);
-    const int blocks = ahead_blocks(h.ahead, h.tiles.blocks(), S::kThreads);
-    k_pk_gemm<EPI, kSplit, S><<<dim3(blocks, splits), S::kThreads, sizeof(tile::Lds<S>), s>>>(h);
-  });
+  tile::with_shape(g.M, g.N, splits, [&](auto shape) { launch_tiles<EPI, kSplit, false, decltype(shape)>(g, splits, s); });
+}
+// Rows farther apart than a tile's 32-bit offsets reach (256 rows of kFarRows
+// elements: 2 GB). Two tile shapes are enough for these: 128 x 128 x 8,192 in
+// 1 / 8 splits 26 / 13 us, as near rows (an output per thread took 704).
+constexpr int kFarRows = 1 << 22;
+template <int EPI, bool kSplit>
+void launch_far(const PkGemm& g, int splits, hipStream_t s) {
+  if (tile::blocks_of<tile::S32x64>(g.M, g.N) * splits <= tile::kCus)
+    launch_tiles<EPI, kSplit, true, tile::S32x64>(g, splits, s);
+  else
+    launch_tiles<EPI, kSplit, true, tile::S128x128>(g, splits, s);
 }
 
 template <int EPI>
@@ -908,22 +913,21 @@ int gemm(const uint16_t* a, int lda, const uint16_t* bt, int ldb, const uint16_t
          int n, int k, int epi, int splits, float* part, hipStream_t s, const AheadPair& ahead = {}) {
   const bool wide = aligned16(c) && ldc % 8 == 0;
   const PkGemm g{a, bt, bias, c, part, 0.0f, lda, ldb, ldc, m, n, k / splits, wide, {}, splits > 1 ? AheadPair{} : ahead};
-  if (lda > kFarRows || ldb > kFarRows) {
-    PkGemm f = g;
-    f.kchunk = k;
-    const dim3 grid((n + 255) / 256, m);
-    switch (epi) {
-      case EPI_NONE: k_pk_gemm_far<EPI_NONE><<<grid, 256, 0, s>>>(f); break;
-      case EPI_BIAS: k_pk_gemm_far<EPI_BIAS><<<grid, 256, 0, s>>>(f); break;
-      default: k_pk_gemm_far<EPI_SWISH><<<grid, 256, 0, s>>>(f); break;
-    }
-  } else if (splits > 1) {
-    launch_gemm<EPI_NONE, true>(g, splits, s);
+  const bool far = lda > kFarRows || ldb > kFarRows;
+  if (splits > 1) {
+    if (far) launch_far<EPI_NONE, true>(g, splits, s);
+    else launch_gemm<EPI_NONE, true>(g, splits, s);
     const dim3 blocks((unsigned)m, (unsigned)((n / 4 + 255) / 256));
     switch (epi) {
       case EPI_NONE: launch_splitk<EPI_NONE>(blocks, part, splits, m, n, bias, c, ldc, s); break;
       case EPI_BIAS: launch_splitk<EPI_BIAS>(blocks, part, splits, m, n, bias, c, ldc, s); break;
       default: launch_splitk<EPI_SWISH>(blocks, part, splits, m, n, bias, c, ldc, s); break;
+    }
+  } else if (far) {
+    switch (epi) {
+      case EPI_NONE: launch_far<EPI_NONE, false>(g, 1, s); break;
+      case EPI_BIAS: launch_far<EPI_BIAS, false>(g, 1, s); break;
+      default: launch_far<EPI_SWISH, false>(g, 1, s); break;
     }
   } else {
     switch (epi) {

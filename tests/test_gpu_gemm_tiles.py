@@ -73,3 +73,43 @@ def test_swish_epilogue_over_the_whole_range(lab, gpu):
     close = (c.double() - want).abs() <= 0.5001 * step
     assert bool((same | close | (tiny & (c.double().abs() < 2.0 ** -126))).all())
     assert int((~same & ~tiny).sum()) <= 64  # ~3 of 2^24 per value off a boundary
+
+
+@pytest.mark.parametrize("m,n,k,splits", [
+    (130, 128, 8192, 1),    # 32 x 64 tiles
+    (130, 128, 8192, 8),
+    (700, 1280, 192, 1),    # 128 x 128 tiles, ragged
+    (700, 1280, 256, 2),
+])
+def test_far_rows_take_the_tiles_and_the_splits(lab, gpu, m, n, k, splits):
+    """Rows of A and then of B farther apart than a tile's 32-bit offsets
+    reach: exact, beside rows that hold NaN past k, and in about the time of
+    near rows (an output per thread took 26 times as long)."""
+    far = (1 << 22) + 8
+
+    def run(a, lda, b, ldb):
+        c = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu)
+        ws = torch.full((splits * m * n,), float("nan"), dtype=torch.float32, device=gpu)
+        times = []
+        for _ in range(6):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            lab._lib.call("lfm25_pk_gemm", a.data_ptr(), lda, b.data_ptr(), ldb, bias.data_ptr(), c.data_ptr(), n, m, n,
+                          k, 1, splits, ws.data_ptr(), torch.cuda.current_stream().cuda_stream)
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end))
+        assert torch.equal(c, want)
+        return min(times)
+
+    def spread(x):
+        y = torch.empty(x.shape[0], far, dtype=torch.bfloat16, device=gpu)
+        y[:, :k] = x
+        y[:, k:k + 64] = float("nan")
+        return y
+
+    a, b, bias = ints(6, (m, k), gpu), ints(7, (n, k), gpu), ints(8, (n,), gpu)
+    want = (a.double() @ b.double().T.contiguous() + bias.double()).to(torch.bfloat16)
+    near = run(a, k, b, k)
+    assert run(spread(a), far, b, k) <= 5 * near
+    assert run(a, k, spread(b), far) <= 5 * near
