@@ -1,11 +1,15 @@
 """The layer programs of csrc/lfm25_layer.hip at the edges of their position
 blocks: attention_context_cache against attention_context and
-append_attention_cache (which the oracle holds elsewhere)."""
+append_attention_cache (which the oracle holds elsewhere), and its context
+inside the interval derived from the oracle's algorithm, which a position
+more or less leaves."""
 
 from __future__ import annotations
 
 import pytest
 import torch
+
+from parity_helpers import attention_interval
 
 pytestmark = pytest.mark.gpu
 
@@ -41,6 +45,13 @@ def test_context_cache_at_block_edges(lab, gpu, past):
     v = nxt.view(8, 2, past + 1, 64)[:, 1].double().abs().amax(dim=(1, 2)).repeat_interleave(128)
     assert bool(((a - b).abs() <= 2.0 ** -8 * b.abs() + 2.0 ** -16 * v).all() | (past > 64) &
                 ((a - b).abs() <= 2.0 ** -7 * b.abs().clamp_min(b.abs().mean())).all())
+    # FP32 roundings on one path: a lane's passes of 512 positions, five over
+    # the lanes, sixteen waves; the sum of the probabilities has fewer
+    rows = nxt.view(8, 2, past + 1, 64).float().cpu().numpy()
+    lo, hi = attention_interval(qkv[:1024].view(16, 64).float().cpu().numpy(), rows[:, 0], rows[:, 1],
+                                24 + (past + 1) // 512)
+    got = tail[1024:].double().cpu().numpy()
+    assert ((got >= lo) & (got <= hi)).all()
 
 
 def test_context_cache_of_a_misaligned_cache(lab, gpu):
